@@ -179,7 +179,7 @@ int plan_group(cqr_ctx* c, cqr_batch* bt, Group& g, bool alloc = true) {
   g.Uinv = s.add(8 * np * bb);
   g.Winv = s.add(8 * np * bb);
   g.LinvT = s.add(8 * np * bb);
-  g.cnt = s.add(8 * nn);
+  g.cnt = s.add(8 * CQR_TREE_FLAGS * nn);
   g.qflags = s.add(8 * nn * (size_t)((b + 15) / 16));
   g.bytes = s.bytes;
   build_order(g);
@@ -218,7 +218,7 @@ int run_group(cqr_ctx* c, cqr_batch* bt, const Group& g, double* A, double* Tt) 
   const int64_t bb = (int64_t)b * b;
   uint64_t* cnt = reinterpret_cast<uint64_t*>(base + g.cnt);
   uint64_t* qf = reinterpret_cast<uint64_t*>(base + g.qflags);
-  CQR_TRY(fill_u64(c, cnt, std::max(g.total_nodes, 1)));
+  CQR_TRY(fill_u64(c, cnt, CQR_TREE_FLAGS * (int64_t)std::max(g.total_nodes, 1)));
   CQR_TRY(fill_u64(c, qf, (int64_t)std::max(g.total_nodes, 1) * ((b + 15) / 16)));
   CQR_TRY(leaf_qr_batched(c, A, g.total_rows, g.total_leaves, g.max_leaf_rows, b, at(g.leafR), at(g.leafT),
                           at(g.leafTau), g.d_bp, np));

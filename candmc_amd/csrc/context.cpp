@@ -293,7 +293,7 @@ int cqr_create(cqr_ctx** ctx, int device) {
       c->num_cu < 1)
     c->num_cu = 256;
   if (hipMalloc(&c->d_flag, sizeof(int)) != hipSuccess ||
-      hipMalloc(&c->d_cnt, sizeof(uint64_t) * CQR_MAX_TREE_NODES * 2) != hipSuccess ||
+      hipMalloc(&c->d_cnt, sizeof(uint64_t) * CQR_TREE_FLAGS * CQR_MAX_TREE_NODES * 2) != hipSuccess ||
       hipMalloc(&c->d_terr, 2 * sizeof(int)) != hipSuccess ||   // [0] timeout flag, [1] poll bound
       hipMalloc(&c->d_qflags, sizeof(uint64_t) * CQR_MAX_TREE_NODES * 8) != hipSuccess ||
       hipMemset(c->d_qflags, 0, sizeof(uint64_t) * CQR_MAX_TREE_NODES * 8) != hipSuccess ||
@@ -301,7 +301,7 @@ int cqr_create(cqr_ctx** ctx, int device) {
       hipHostMalloc(&c->h_pin, 64 * sizeof(double), hipHostMallocDefault) != hipSuccess ||
       hipEventCreateWithFlags(&c->ev_host, hipEventDisableTiming) != hipSuccess ||
       hipMemset(c->d_terr, 0, 2 * sizeof(int)) != hipSuccess ||
-      hipMemset(c->d_cnt, 0, sizeof(uint64_t) * CQR_MAX_TREE_NODES * 2) != hipSuccess ||
+      hipMemset(c->d_cnt, 0, sizeof(uint64_t) * CQR_TREE_FLAGS * CQR_MAX_TREE_NODES * 2) != hipSuccess ||
       hipMemset(c->d_flag, 0, sizeof(int)) != hipSuccess ||
       hipEventCreateWithFlags(&c->ev_fork, hipEventDisableTiming) != hipSuccess ||
       hipEventCreateWithFlags(&c->ev_join, hipEventDisableTiming) != hipSuccess ||

@@ -35,7 +35,7 @@ struct cqr_ctx {
   int check_finite = 0;
   int64_t leaf_rows = 0;        // 0 = automatic
   int* d_flag = nullptr;        // device flag for non-finite scans / tree timeouts
-  uint64_t* d_cnt = nullptr;    // column counters: tree nodes, then (second half) leaves
+  uint64_t* d_cnt = nullptr;    // progress words: tree nodes, then (second half) leaves
   int* d_terr = nullptr;        // set by a tree node whose wait for a child timed out
   uint64_t* d_qflags = nullptr; // per (node, column block) flags of construct_Q1
   uint64_t* d_sflags = nullptr; // per 128-row block flags of the one-launch triangular solve
@@ -234,9 +234,10 @@ __device__ inline int seg_find(const BatchSeg* s, int nseg, int idx) {
 }
 
 #define CQR_MAX_TREE_NODES 8192
+#define CQR_TREE_FLAGS 8           // progress words per tree node and per leaf: one per 16-column block
 #define CQR_TRSM_MAX_BLOCKS 4096   // 128-row blocks of the one-launch triangular solve
 
-// Column-pipelined tree over all levels (ptree_kernel.hip): node outputs R
+// Pipelined tree over all levels (ptree_kernel.hip): node outputs R
 // in nodeR (nnodes×b×b), V2/T/tau per node in forward level order.
 int leaf_tree(cqr_ctx* c, double* A, int64_t lda, int64_t m, int L, int b, double* leafR, double* leafT,
               double* leafTau, double* nodeR, double* V2, double* T, double* tau, int nnodes);
@@ -268,6 +269,10 @@ int hr_core_batched(cqr_ctx* c, const BatchProb* bp, int nprob, const double* Y,
 int gemm_f64_batched_prob(cqr_ctx* c, int ta, int tb, int m, int n, int k, double alpha, const BMat& A, int smA,
                           const BMat& B, int smB, double beta, const BMat& C, int smC, int nprob, const BatchProb* bp,
                           int64_t prow, int m_prob, int max_m);
+
+// Leaves of 64 < b ≤ 128 columns and at most 256 rows (ptree_kernel.hip)
+int leaf16(cqr_ctx* c, double* A, int64_t lda, int64_t m, int L, int64_t rows, int b, double* R, double* T, double* tau,
+           const BatchProb* bp, int nprob);
 
 // Kernel launchers (tsqr_kernels.hip)
 int leaf_qr(cqr_ctx* c, double* A, int64_t lda, int64_t m, int L, int b, double* R, double* T,

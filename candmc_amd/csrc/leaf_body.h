@@ -1,4 +1,4 @@
-// Leaf QR body shared by the leaf kernel and the fused leaf + tree kernel.
+// Leaf QR body for panels of at most 64 columns (wider ones: panel16.h).
 #pragma once
 
 #include "cqr_device.h"
@@ -17,17 +17,11 @@ __device__ __forceinline__ int64_t leaf_off(int64_t l, int64_t m, int64_t L) { r
 // The dot products against the already-finished columns are the Gram
 // entries V(:,j)ᵀv_i that give the compact-WY T at the end.
 // ---------------------------------------------------------------------------
-//
-// With `lcnt` set, the leaf also publishes its R while it runs: column i of
-// R (rows ≤ i) is final once its reflector exists, so the owner wave stores
-// it at once with device-coherent stores; after every eighth column all
-// waves wait for their stores and lcnt[leaf] = epoch·256 + (columns done)
-// tells a consumer in the same launch that those columns may be read.
 template <int WAVES, int CPW, int RPL>
 __device__ __forceinline__ void leaf_qr_body(double* __restrict__ A, int64_t lda, int64_t m, int L, int b,
                                     double* __restrict__ Rout, double* __restrict__ Tout,
                                     double* __restrict__ tauout, const BatchProb* __restrict__ bp, int nprob,
-                                    int gleaf, double* smem, uint64_t* __restrict__ lcnt, uint64_t epoch) {
+                                    int gleaf, double* smem) {
   constexpr int NT = 64 * WAVES;
   int leaf = gleaf;
   if (bp) {                      // batched: A is the group's base, the problem's block at aoff
@@ -121,20 +115,9 @@ __device__ __forceinline__ void leaf_qr_body(double* __restrict__ A, int64_t lda
           vb[row] = row > i ? a[cl][s] : (row == i ? 1.0 : 0.0);
         }
         if (lane == 0) stau[i] = h.tau;
-        if (lcnt) {
-#pragma unroll
-          for (int s = 0; s < RPL; ++s) {
-            const int row = lane + 64 * s;
-            if (row <= i) store_coherent(Rl + row + (int64_t)i * b, a[cl][s]);
-          }
-        }
       }
     }
-    // before a block of eight columns is published, every owner's R stores
-    // have completed
-    if (lcnt && ((i & 7) == 7 || i + 1 == b)) wait_memory();
     __syncthreads();
-    if (lcnt && tid == 0 && ((i & 7) == 7 || i + 1 == b)) flag_store(lcnt + gleaf, epoch * 256 + (uint64_t)(i + 1));
     const double tau = stau[i];
     double v[RPL];
 #pragma unroll

@@ -1,0 +1,453 @@
+// Sixteen-column panel steps shared by the leaf QR and the tree nodes.
+//
+// One wave holds a 16-column strip of the matrix as 16×16 tiles in the
+// layout of a v_mfma_f64_16x16x4f64 result: lane l, value v of a tile holds
+// tile row "i = (l >> 4) + 4v" of column l & 15.  A tile in this layout is
+// directly the B operand of the next product (value v is its k-slice v), so
+// the strip never leaves its registers.  Which matrix row tile row i stands
+// for is free as long as every tile of a launch agrees: `PERM` strips map
+// (g = l >> 4, v) to row 4g + v, so that a lane's four values are 32
+// contiguous bytes of a column; the pivot tiles of tree nodes use i itself.
+//
+// The panel is factored by the wave that owns its strip, without LDS and
+// without barriers: in a column step every lane needs column jj's value of
+// its own row, which the DPP row broadcast of v_fmac_f64_dpp supplies for
+// free, so the sixteen dot products x·a_c (‖x‖² among them) and the rank-1
+// update are one FMA per value.  (Measured on gfx950: the broadcast FMA
+// issues in 4 cycles, as the plain one does.)
+#pragma once
+
+#include "cqr_device.h"
+
+namespace cqr {
+
+constexpr int P16 = 16;               // panel width
+constexpr int P16_LD = 17;            // pitch of a 16×16 tile in LDS (row-major)
+constexpr int P16_TILE = 16 * P16_LD;
+
+// The tile stored row-major in LDS, in tile layout, and back.
+__device__ __forceinline__ dbl4 p16_load(const double* __restrict__ X, int lane) {
+  const double* xp = X + (lane >> 4) * P16_LD + (lane & 15);
+  return dbl4{xp[0], xp[4 * P16_LD], xp[8 * P16_LD], xp[12 * P16_LD]};
+}
+__device__ __forceinline__ void p16_store(double* __restrict__ X, const dbl4& y, int lane) {
+  double* xp = X + (lane >> 4) * P16_LD + (lane & 15);
+#pragma unroll
+  for (int v = 0; v < 4; ++v) xp[4 * v * P16_LD] = y[v];
+}
+
+// s[v] += x_t[v](column J)·x_t[v] over four tiles.  The leading s_nop covers
+// the two wait states a DPP source needs after a VALU write.
+template <int J>
+__device__ __forceinline__ void p16_dot4(double (&s)[4], const dbl4& a, const dbl4& b, const dbl4& c, const dbl4& d) {
+  asm("s_nop 1\n"
+      "v_fmac_f64_dpp %0, %4, %4 row_newbcast:%20 row_mask:0xf bank_mask:0xf\n"
+      "v_fmac_f64_dpp %1, %5, %5 row_newbcast:%20 row_mask:0xf bank_mask:0xf\n"
+      "v_fmac_f64_dpp %2, %6, %6 row_newbcast:%20 row_mask:0xf bank_mask:0xf\n"
+      "v_fmac_f64_dpp %3, %7, %7 row_newbcast:%20 row_mask:0xf bank_mask:0xf\n"
+      "v_fmac_f64_dpp %0, %8, %8 row_newbcast:%20 row_mask:0xf bank_mask:0xf\n"
+      "v_fmac_f64_dpp %1, %9, %9 row_newbcast:%20 row_mask:0xf bank_mask:0xf\n"
+      "v_fmac_f64_dpp %2, %10, %10 row_newbcast:%20 row_mask:0xf bank_mask:0xf\n"
+      "v_fmac_f64_dpp %3, %11, %11 row_newbcast:%20 row_mask:0xf bank_mask:0xf\n"
+      "v_fmac_f64_dpp %0, %12, %12 row_newbcast:%20 row_mask:0xf bank_mask:0xf\n"
+      "v_fmac_f64_dpp %1, %13, %13 row_newbcast:%20 row_mask:0xf bank_mask:0xf\n"
+      "v_fmac_f64_dpp %2, %14, %14 row_newbcast:%20 row_mask:0xf bank_mask:0xf\n"
+      "v_fmac_f64_dpp %3, %15, %15 row_newbcast:%20 row_mask:0xf bank_mask:0xf\n"
+      "v_fmac_f64_dpp %0, %16, %16 row_newbcast:%20 row_mask:0xf bank_mask:0xf\n"
+      "v_fmac_f64_dpp %1, %17, %17 row_newbcast:%20 row_mask:0xf bank_mask:0xf\n"
+      "v_fmac_f64_dpp %2, %18, %18 row_newbcast:%20 row_mask:0xf bank_mask:0xf\n"
+      "v_fmac_f64_dpp %3, %19, %19 row_newbcast:%20 row_mask:0xf bank_mask:0xf"
+      : "+&v"(s[0]), "+&v"(s[1]), "+&v"(s[2]), "+&v"(s[3])
+      : "v"(a[0]), "v"(a[1]), "v"(a[2]), "v"(a[3]), "v"(b[0]), "v"(b[1]), "v"(b[2]), "v"(b[3]), "v"(c[0]), "v"(c[1]),
+        "v"(c[2]), "v"(c[3]), "v"(d[0]), "v"(d[1]), "v"(d[2]), "v"(d[3]), "n"(J));
+}
+
+// N rows of the pivot tile (N ≤ 4): s[v & 1] += x_v(column J)·x_v, and
+// x_v += x_v(column J)·f.
+#define P16_BC " row_newbcast:%c[j] row_mask:0xf bank_mask:0xf\n"
+template <int J, int N>
+__device__ __forceinline__ void p16_dotrows(double (&s)[2], const double* x) {
+  if constexpr (N == 1)
+    asm("s_nop 1\n v_fmac_f64_dpp %0, %2, %2" P16_BC : "+&v"(s[0]), "+&v"(s[1]) : "v"(x[0]), [j] "n"(J));
+  else if constexpr (N == 2)
+    asm("s_nop 1\n v_fmac_f64_dpp %0, %2, %2" P16_BC "v_fmac_f64_dpp %1, %3, %3" P16_BC
+        : "+&v"(s[0]), "+&v"(s[1]) : "v"(x[0]), "v"(x[1]), [j] "n"(J));
+  else if constexpr (N == 3)
+    asm("s_nop 1\n v_fmac_f64_dpp %0, %2, %2" P16_BC "v_fmac_f64_dpp %1, %3, %3" P16_BC "v_fmac_f64_dpp %0, %4, %4" P16_BC
+        : "+&v"(s[0]), "+&v"(s[1]) : "v"(x[0]), "v"(x[1]), "v"(x[2]), [j] "n"(J));
+  else
+    asm("s_nop 1\n v_fmac_f64_dpp %0, %2, %2" P16_BC "v_fmac_f64_dpp %1, %3, %3" P16_BC "v_fmac_f64_dpp %0, %4, %4" P16_BC
+        "v_fmac_f64_dpp %1, %5, %5" P16_BC
+        : "+&v"(s[0]), "+&v"(s[1]) : "v"(x[0]), "v"(x[1]), "v"(x[2]), "v"(x[3]), [j] "n"(J));
+}
+template <int J, int N>
+__device__ __forceinline__ void p16_axpyrows(double* x, double f) {
+  if constexpr (N == 1)
+    asm("s_nop 1\n v_fmac_f64_dpp %0, %0, %[f]" P16_BC : "+&v"(x[0]) : [f] "v"(f), [j] "n"(J));
+  else if constexpr (N == 2)
+    asm("s_nop 1\n v_fmac_f64_dpp %0, %0, %[f]" P16_BC "v_fmac_f64_dpp %1, %1, %[f]" P16_BC
+        : "+&v"(x[0]), "+&v"(x[1]) : [f] "v"(f), [j] "n"(J));
+  else if constexpr (N == 3)
+    asm("s_nop 1\n v_fmac_f64_dpp %0, %0, %[f]" P16_BC "v_fmac_f64_dpp %1, %1, %[f]" P16_BC "v_fmac_f64_dpp %2, %2, %[f]" P16_BC
+        : "+&v"(x[0]), "+&v"(x[1]), "+&v"(x[2]) : [f] "v"(f), [j] "n"(J));
+  else
+    asm("s_nop 1\n v_fmac_f64_dpp %0, %0, %[f]" P16_BC "v_fmac_f64_dpp %1, %1, %[f]" P16_BC "v_fmac_f64_dpp %2, %2, %[f]" P16_BC
+        "v_fmac_f64_dpp %3, %3, %[f]" P16_BC
+        : "+&v"(x[0]), "+&v"(x[1]), "+&v"(x[2]), "+&v"(x[3]) : [f] "v"(f), [j] "n"(J));
+}
+
+// a[v] += a[v](column J)·f (one tile in place)
+template <int J>
+__device__ __forceinline__ void p16_axpy1(dbl4& a, double f) {
+  double a0 = a[0], a1 = a[1], a2 = a[2], a3 = a[3];
+  asm("s_nop 1\n"
+      "v_fmac_f64_dpp %0, %0, %4 row_newbcast:%5 row_mask:0xf bank_mask:0xf\n"
+      "v_fmac_f64_dpp %1, %1, %4 row_newbcast:%5 row_mask:0xf bank_mask:0xf\n"
+      "v_fmac_f64_dpp %2, %2, %4 row_newbcast:%5 row_mask:0xf bank_mask:0xf\n"
+      "v_fmac_f64_dpp %3, %3, %4 row_newbcast:%5 row_mask:0xf bank_mask:0xf"
+      : "+&v"(a0), "+&v"(a1), "+&v"(a2), "+&v"(a3)
+      : "v"(f), "n"(J));
+  a = dbl4{a0, a1, a2, a3};
+}
+
+// a[v] += a[v](column J)·f, b likewise (two tiles in place).
+template <int J>
+__device__ __forceinline__ void p16_axpy2(dbl4& a, dbl4& b, double f) {
+  double a0 = a[0], a1 = a[1], a2 = a[2], a3 = a[3], b0 = b[0], b1 = b[1], b2 = b[2], b3 = b[3];
+  asm("s_nop 1\n"
+      "v_fmac_f64_dpp %0, %0, %8 row_newbcast:%9 row_mask:0xf bank_mask:0xf\n"
+      "v_fmac_f64_dpp %1, %1, %8 row_newbcast:%9 row_mask:0xf bank_mask:0xf\n"
+      "v_fmac_f64_dpp %2, %2, %8 row_newbcast:%9 row_mask:0xf bank_mask:0xf\n"
+      "v_fmac_f64_dpp %3, %3, %8 row_newbcast:%9 row_mask:0xf bank_mask:0xf\n"
+      "v_fmac_f64_dpp %4, %4, %8 row_newbcast:%9 row_mask:0xf bank_mask:0xf\n"
+      "v_fmac_f64_dpp %5, %5, %8 row_newbcast:%9 row_mask:0xf bank_mask:0xf\n"
+      "v_fmac_f64_dpp %6, %6, %8 row_newbcast:%9 row_mask:0xf bank_mask:0xf\n"
+      "v_fmac_f64_dpp %7, %7, %8 row_newbcast:%9 row_mask:0xf bank_mask:0xf"
+      : "+&v"(a0), "+&v"(a1), "+&v"(a2), "+&v"(a3), "+&v"(b0), "+&v"(b1), "+&v"(b2), "+&v"(b3)
+      : "v"(f), "n"(J));
+  a = dbl4{a0, a1, a2, a3};
+  b = dbl4{b0, b1, b2, b3};
+}
+
+// acc += z(lane C of the row)·t
+template <int C>
+__device__ __forceinline__ void p16_fma_bc(double& acc, double z, double t) {
+  asm("v_fmac_f64_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf" : "+&v"(acc) : "v"(z), "v"(t), "n"(C));
+}
+
+// sqrt and the two reciprocals of dlarfg for ss = ‖x‖² in (2^-200, 2^200)
+// and |alpha| < 2^200: beta = −sign(alpha)·sqrt(alpha² + ss) by the
+// Goldschmidt iteration from the hardware's reciprocal square root with two
+// residual corrections; no operand scaling is needed in this range.
+__device__ __forceinline__ void p16_larfg(double alpha, double ss, double& beta, double& tau, double& scal, double& rb) {
+  const double x = fma(alpha, alpha, ss);
+  const double y = __builtin_amdgcn_rsq(x);
+  double g = x * y, h = 0.5 * y;
+  const double r = fma(-h, g, 0.5);
+  h = fma(h, r, h);
+  g = fma(g, r, g);
+  g = fma(fma(-g, g, x), h, g);
+  g = fma(fma(-g, g, x), h, g);
+  beta = -copysign(g, alpha);
+  // 1/beta from the refined reciprocal root h ≈ 1/(2g)
+  double q = h + h;
+  q = fma(q, fma(-g, q, 1.0), q);
+  rb = copysign(q, beta);
+  scal = recip_nr(alpha - beta);
+  tau = (beta - alpha) * rb;
+}
+
+// One panel: RT tiles below the pivot tile, the pivot tile's sixteen rows
+// (row q of every column, the same in all four lane groups), and per lane
+// (column c = lane & 15) its reflector's tau and the scale still to be
+// applied to its vector.
+//   NODE = false: the pivot tile's rows below the diagonal belong to the
+//     reflectors (a leaf; tile rows map as 4g + v).
+//   NODE = true:  the pivot tile is the top triangle of a stacked pair: a
+//     reflector is [e_jj; x] and only row jj takes part (rows map as g + 4v).
+// LDS: Zs, a 16×16 tile whose row J receives −tau_J·v_qᵀv_J (q < J) and in
+// the end the panel's compact-WY T, transposed; Vs (RT tiles), where the
+// strip is kept for the slow path and the scaled vectors are left; Ds (one
+// tile), the pivot tile before and after.
+template <int RT, bool NODE>
+struct Panel16 {
+  // the tiles [H, RT) are skipped as a whole once they are zero
+  static constexpr int H = RT > 8 ? 8 : RT > 4 ? 4 : RT;
+  double pr[P16];          // pivot rows
+  double tau, scale;
+  double ssv, alv, smax;   // what decides the fast range: ‖x‖², alpha per column, largest |dot|
+
+  // tile row that holds matrix row q of the pivot tile
+  __device__ static constexpr int trow_of(int q) { return NODE ? q : (q >> 2) + 4 * (q & 3); }
+
+  template <int J, int T0, int T1>
+  __device__ static __forceinline__ void dots(double (&s4)[4], const dbl4 (&a)[RT]) {
+    const dbl4 zero = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int t = T0; t < T1; t += 4)
+      p16_dot4<J>(s4, a[t], t + 1 < T1 ? a[t + 1 < T1 ? t + 1 : 0] : zero, t + 2 < T1 ? a[t + 2 < T1 ? t + 2 : 0] : zero,
+                  t + 3 < T1 ? a[t + 3 < T1 ? t + 3 : 0] : zero);
+  }
+  template <int J, int T0, int T1>
+  __device__ static __forceinline__ void axpys(dbl4 (&a)[RT], double f) {
+#pragma unroll
+    for (int t = T0; t < T1; t += 2) {
+      if (t + 1 < T1) p16_axpy2<J>(a[t], a[t + 1 < T1 ? t + 1 : t], f);
+      else p16_axpy1<J>(a[t], f);
+    }
+  }
+
+  // Column J.  Exact in the fast range (checked for all columns at the end:
+  // outside it the panel is redone by slow()).
+  template <int J>
+  __device__ __forceinline__ void column(dbl4 (&a)[RT], int nact, double* __restrict__ Zc) {
+    // an opaque copy: the code is not duplicated per number of active tiles,
+    // and no lane mask lives across columns
+    int lane;
+    asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n v_mbcnt_hi_u32_b32 %0, -1, %0" : "=&v"(lane), "+s"(nact));
+    const int c = lane & 15;
+    constexpr int N = P16 - 1 - J;              // pivot rows below row J
+    double s4[4] = {0.0, 0.0, 0.0, 0.0}, d2[2] = {0.0, 0.0};
+    dots<J, 0, H>(s4, a);
+    if constexpr (RT > H)
+      if (__builtin_expect(nact > H, 1)) dots<J, H, RT>(s4, a);
+    double s = (s4[0] + s4[1]) + (s4[2] + s4[3]);
+    if constexpr (!NODE) {
+#pragma unroll
+      for (int q = 0; q + 4 <= N; q += 4) p16_dotrows<J, 4>(d2, pr + J + 1 + q);
+      if constexpr (N % 4 != 0) p16_dotrows<J, N % 4>(d2, pr + P16 - N % 4);
+    }
+    s = xr_cross_rows(s);
+    if constexpr (!NODE) s += d2[0] + d2[1];
+    const double p = pr[J];
+    const double ss = readlane_d(s, J), alpha = readlane_d(p, J);
+    double beta, tj, scal, rb;
+    p16_larfg(alpha, ss, beta, tj, scal, rb);
+    const double wv = fma(scal, s, p);          // v_Jᵀ·(column c), v_J = [1; scal·x]
+    const double f = c > J ? wv * rb : 0.0;     // −tau·scal = 1/beta
+    axpys<J, 0, H>(a, f);
+    asm volatile("" : "+s"(nact));
+    if constexpr (RT > H)
+      if (__builtin_expect(nact > H, 1)) axpys<J, H, RT>(a, f);
+    if constexpr (!NODE) {
+#pragma unroll
+      for (int q = 0; q + 4 <= N; q += 4) p16_axpyrows<J, 4>(pr + J + 1 + q, f);
+      if constexpr (N % 4 != 0) p16_axpyrows<J, N % 4>(pr + P16 - N % 4, f);
+    }
+    pr[J] = c > J ? fma(-tj, wv, p) : (c == J ? beta : p);
+    Zc[J * P16_LD] = wv * scale * -tj;          // four lanes, one value
+    smax = fmax(smax, fabs(s));
+    ssv = c == J ? s : ssv;
+    alv = c == J ? p : alv;
+    tau = c == J ? tj : tau;
+    scale = c == J ? scal : scale;
+  }
+
+  // The whole panel with dlarfg's general semantics (rescaling, zero and
+  // non-finite columns), in LDS: nt tiles in Vs, the pivot tile in Ds.
+  __device__ __forceinline__ static void slow(double* Vs, double* Ds, double* Zs, int nt, int nb, double& tau_out) {
+    const int lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
+    auto sync = []() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup"); };
+    // element v of this lane's column in tile t (t < 0: the pivot tile)
+    auto at = [&](int t, int v) -> double& { return (t < 0 ? Ds : Vs + t * P16_TILE)[(g + 4 * v) * P16_LD + c]; };
+    auto pivot_row = [&](int v) { return NODE ? g + 4 * v : 4 * g + v; };
+    const int t0 = NODE ? 0 : -1;
+    double tau = 0.0;
+#pragma unroll 1
+    for (int j = 0; j < nb; ++j) {
+      const int src = (lane & 48) | j;
+      const int jr = trow_of(j);
+      const double p = Ds[jr * P16_LD + c];
+      const double alpha = readlane_d(p, j);
+      auto below = [&](int t, int v) { return t >= 0 || pivot_row(v) > j; };
+      double mx = 0.0;
+#pragma unroll 1
+      for (int t = t0; t < nt; ++t)
+        for (int v = 0; v < 4; ++v)
+          if (below(t, v)) mx = fmax(mx, fabs(at(t, v)));
+      mx = fmax(mx, __shfl_xor(mx, 16));
+      mx = readlane_d(fmax(mx, __shfl_xor(mx, 32)), j);
+      double s2 = 0.0;
+#pragma unroll 1
+      for (int t = t0; t < nt; ++t)
+        for (int v = 0; v < 4; ++v)
+          if (below(t, v)) {
+            const double x = at(t, v) / mx;
+            s2 += x * x;
+          }
+      s2 = readlane_d(xr_cross_rows(s2), j);
+      const Reflector h = dlarfg_scalar(alpha, mx == 0.0 ? 0.0 : mx * sqrt(s2));
+      if (c == j && h.tau != 0.0)
+  #pragma unroll 1
+      for (int t = t0; t < nt; ++t)
+          for (int v = 0; v < 4; ++v)
+            if (below(t, v)) {
+              double x = at(t, v);
+              for (int k = 0; k < h.knt; ++k) x *= 0x1p969;
+              at(t, v) = x * h.scal;
+            }
+      sync();
+      double s = 0.0;
+#pragma unroll 1
+      for (int t = t0; t < nt; ++t)
+        for (int v = 0; v < 4; ++v) {
+          const double x = __shfl(at(t, v), src);
+          if (below(t, v)) s += x * at(t, v);
+        }
+      const double wv = p + xr_cross_rows(s), f = h.tau * wv;
+#pragma unroll 1
+      for (int t = t0; t < nt; ++t)
+        for (int v = 0; v < 4; ++v) {
+          const double x = __shfl(at(t, v), src);
+          if (c > j && below(t, v)) at(t, v) -= f * x;
+        }
+      if (g == 0) {
+        Ds[jr * P16_LD + c] = c > j ? p - f : (c == j ? h.beta : p);
+        Zs[j * P16_LD + c] = c < j ? -h.tau * wv : 0.0;
+      }
+      if (c == j) tau = h.tau;
+      sync();
+    }
+    tau_out = tau;
+  }
+
+  template <int J, int Q = 0>
+  __device__ static __forceinline__ void tsum(double& acc, const double& z, const double (&trow)[P16]) {
+    if constexpr (Q < J) {
+      p16_fma_bc<Q>(acc, z, trow[Q]);
+      tsum<J, Q + 1>(acc, z, trow);
+    }
+  }
+  // T(0:J, J) = −tau_J·T(0:J, 0:J)·(v_qᵀv_J)_q, T(J, J) = tau_J, from column J on
+  template <int J>
+  __device__ __forceinline__ void tcols(double (&trow)[P16], const double (&z)[P16], int c) const {
+    if constexpr (J < P16) {
+      double acc = c == J ? tau : 0.0;
+      asm("s_nop 1" : "+v"(acc) : "v"(z[J]));
+      tsum<J>(acc, z[J], trow);
+      trow[J] = acc;
+      tcols<J + 1>(trow, z, c);
+    }
+  }
+
+  // Factors the first nb columns of the strip (D; a); nact tiles of `a` may
+  // be nonzero.  On return Vs holds the vectors scaled as dlarfg's (every
+  // tile that can be nonzero, and zeros up to tile H), Ds and D the pivot
+  // tile (R rows and, for a leaf, the vectors below its diagonal) and Zs the
+  // panel's T, transposed; `a` is left unscaled.
+  __device__ __forceinline__ void factor(dbl4& D, dbl4 (&a)[RT], int nact, int nb, int lane, double* Zs, double* Vs,
+                                         double* Ds) {
+    const int c = lane & 15;
+    tau = 0.0;
+    scale = 1.0;
+    ssv = alv = 1.0;
+    smax = 0.0;
+    // the strip may come straight from MFMAs, whose results the inline VALU
+    // code below must not read before they land
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("s_nop 15\n s_nop 15\n s_nop 15");
+    __builtin_amdgcn_sched_barrier(0);
+    // kept for the slow path: straight-line columns with one test at the end
+    // cost less than a way out of every column
+    p16_store(Ds, D, lane);
+#pragma unroll
+    for (int t = 0; t < RT; ++t)
+      if (t < H || nact > H) p16_store(Vs + t * P16_TILE, a[t], lane);
+    double* Zc = Zs + c;
+#pragma unroll
+    for (int q = 0; q < P16; ++q) pr[q] = Ds[trow_of(q) * P16_LD + c];
+    if (nb < P16)
+      for (int q = nb; q < P16; ++q) Zc[q * P16_LD] = 0.0;
+#define P16_STEP(J)                 \
+  asm volatile("" : "+s"(nb));      \
+  if (J == 0 || __builtin_expect(J < nb, 1)) column<J>(a, nact, Zc);
+    P16_STEP(0) P16_STEP(1) P16_STEP(2) P16_STEP(3) P16_STEP(4) P16_STEP(5) P16_STEP(6) P16_STEP(7)
+    P16_STEP(8) P16_STEP(9) P16_STEP(10) P16_STEP(11) P16_STEP(12) P16_STEP(13) P16_STEP(14) P16_STEP(15)
+#undef P16_STEP
+    // the fast range: ‖x‖² in (2^-200, 2^200), |alpha| < 2^200, dots far from
+    // overflow; a NaN or infinity fails it
+    if (__builtin_amdgcn_ballot_w64(!(ssv > 0x1p-200 && ssv < 0x1p200 && fabs(alv) < 0x1p200 && smax < 0x1p800)) != 0) {
+      slow(Vs, Ds, Zs, nact > H ? RT : H, nb, tau);
+    } else {
+#pragma unroll
+      for (int t = 0; t < RT; ++t)
+        if (t < H || nact > H) p16_store(Vs + t * P16_TILE, a[t] * scale, lane);
+#pragma unroll
+      for (int q = 0; q < P16; ++q) Ds[trow_of(q) * P16_LD + c] = !NODE && q > c ? pr[q] * scale : pr[q];
+    }
+    D = p16_load(Ds, lane);
+    double z[P16], trow[P16];
+#pragma unroll
+    for (int q = 0; q < P16; ++q) z[q] = Zc[q * P16_LD];
+    tcols<0>(trow, z, c);
+#pragma unroll
+    for (int q = 0; q < P16; ++q) Zc[q * P16_LD] = trow[q];
+  }
+};
+
+// Products with a published panel: Vk holds its vectors as 16×16 tiles in
+// LDS (row-major, tile row i, pitch P16_LD), a[0..N) the caller's strip.
+// acc (16×16) += Σ_t V_tᵀ·a_t over tiles t < nact (tiles past nact are zero).
+template <int N>
+__device__ __forceinline__ dbl4 p16_vta(const double* __restrict__ Vk, const dbl4 (&a)[N], int nact, dbl4 acc, int lane) {
+  const double* vp = Vk + (lane >> 4) * P16_LD + (lane & 15);
+  dbl4 acc2 = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+  for (int q = 0; q < (N + 3) / 4; ++q)
+    if (q == 0 || 4 * q < nact) {
+#pragma unroll
+      for (int t = 4 * q; t < 4 * q + 4; ++t)
+        if (t < N) {
+#pragma unroll
+          for (int v = 0; v < 4; ++v) {
+            const double x = vp[t * P16_TILE + 4 * v * P16_LD];
+            if (v & 1) acc2 = __builtin_amdgcn_mfma_f64_16x16x4f64(x, a[t][v], acc2, 0, 0, 0);
+            else acc = __builtin_amdgcn_mfma_f64_16x16x4f64(x, a[t][v], acc, 0, 0, 0);
+          }
+        }
+      __builtin_amdgcn_sched_barrier(0);   // sixteen operand loads ahead, no more registers than that
+    }
+  return acc + acc2;
+}
+
+// a_t += V_t·u over tiles t < nact (u: 16×16, tile layout).
+template <int N>
+__device__ __forceinline__ void p16_vu(const double* __restrict__ Vk, dbl4 (&a)[N], int nact, const dbl4& u, int lane) {
+  const double* vp = Vk + (lane & 15) * P16_LD + (lane >> 4);
+#pragma unroll
+  for (int q = 0; q < (N + 3) / 4; ++q)
+    if (q == 0 || 4 * q < nact) {
+      // four tiles' chains interleaved: consecutive MFMAs are independent
+#pragma unroll
+      for (int v = 0; v < 4; ++v)
+#pragma unroll
+        for (int t = 4 * q; t < 4 * q + 4; ++t)
+          if (t < N) a[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(vp[t * P16_TILE + 4 * v], u[v], a[t], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+}
+
+// X·y for a 16×16 X in LDS, row-major (y: tile layout).
+__device__ __forceinline__ dbl4 p16_xy(const double* __restrict__ X, const dbl4& y, dbl4 acc, int lane) {
+  const double* xp = X + (lane & 15) * P16_LD + (lane >> 4);
+#pragma unroll
+  for (int v = 0; v < 4; ++v) acc = __builtin_amdgcn_mfma_f64_16x16x4f64(xp[4 * v], y[v], acc, 0, 0, 0);
+  return acc;
+}
+// The compact-WY T of a factorization advancing by 16-column panels, kept in
+// LDS as 16×16 tiles (transposed, one slot per pair i ≤ k).  Wave i owns tile
+// row i.  In step k (after its barrier) wave j < k leaves the Gram tile
+// V_kᵀV_j in slot (j, k); in step k + 1 wave i < k forms
+//   T(i,k)ᵀ = −T_kkᵀ·Σ_{i≤j<k} (V_kᵀV_j)·T(i,j)ᵀ
+// from those tiles, and in step k + 2, when every wave has read them, puts it
+// into slot (i, k), where only wave i needs it again.
+__device__ __forceinline__ int p16_slot(int i, int k) { return (k * (k + 1) / 2 + i) * P16_TILE; }
+
+__device__ __forceinline__ dbl4 p16_tcol(const double* __restrict__ S, int i, int k, int lane) {
+  dbl4 x = {0.0, 0.0, 0.0, 0.0};
+  for (int j = i; j < k; ++j) x = p16_xy(S + p16_slot(j, k), p16_load(S + p16_slot(i, j), lane), x, lane);
+  const dbl4 zero = {0.0, 0.0, 0.0, 0.0};
+  return -p16_xy(S + p16_slot(k, k), x, zero, lane);
+}
+
+}  // namespace cqr

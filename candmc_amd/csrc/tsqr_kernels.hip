@@ -22,7 +22,8 @@ namespace cqr {
     for (int rr = (int)(threadIdx.x & 63); rr < (b); rr += 64)
 
 // ---------------------------------------------------------------------------
-// K1: leaf QR, one workgroup per leaf (body in leaf_body.h).
+// K1: leaf QR for b ≤ 64, one workgroup per leaf (body in leaf_body.h; wider
+// panels: leaf16 in ptree_kernel.hip).
 // ---------------------------------------------------------------------------
 template <int WAVES, int CPW, int RPL>
 __global__ void __launch_bounds__(64 * WAVES)
@@ -30,7 +31,7 @@ leaf_qr_kernel(double* __restrict__ A, int64_t lda, int64_t m, int L, int b,
                double* __restrict__ Rout, double* __restrict__ Tout, double* __restrict__ tauout,
                const BatchProb* __restrict__ bp, int nprob) {
   extern __shared__ double smem[];
-  leaf_qr_body<WAVES, CPW, RPL>(A, lda, m, L, b, Rout, Tout, tauout, bp, nprob, blockIdx.x, smem, nullptr, 0);
+  leaf_qr_body<WAVES, CPW, RPL>(A, lda, m, L, b, Rout, Tout, tauout, bp, nprob, blockIdx.x, smem);
 }
 
 // Packed column-major triangles in LDS: upper (r ≤ c) and strictly upper.
@@ -820,8 +821,7 @@ int leaf_qr_batched(cqr_ctx* c, double* Abase, int64_t total_m, int L, int64_t r
                                   : leaf_launch<8, 4, 16>(c, Abase, 0, total_m, L, b, R, T, tau, bp, nprob);
   if (b <= 64) return rows <= 256 ? leaf_launch<8, 8, 4>(c, Abase, 0, total_m, L, b, R, T, tau, bp, nprob)
                                   : leaf_launch<8, 8, 8>(c, Abase, 0, total_m, L, b, R, T, tau, bp, nprob);
-  return rows <= 128 ? leaf_launch<16, 8, 2>(c, Abase, 0, total_m, L, b, R, T, tau, bp, nprob)
-                     : leaf_launch<16, 8, 4>(c, Abase, 0, total_m, L, b, R, T, tau, bp, nprob);
+  return leaf16(c, Abase, 0, total_m, L, rows, b, R, T, tau, bp, nprob);
 }
 
 int leaf_qr(cqr_ctx* c, double* A, int64_t lda, int64_t m, int L, int b, double* R, double* T,
@@ -833,10 +833,7 @@ int leaf_qr(cqr_ctx* c, double* A, int64_t lda, int64_t m, int L, int b, double*
                                   : leaf_launch<8, 4, 16>(c, A, lda, m, L, b, R, T, tau);
   if (b <= 64) return rows <= 256 ? leaf_launch<8, 8, 4>(c, A, lda, m, L, b, R, T, tau)
                                   : leaf_launch<8, 8, 8>(c, A, lda, m, L, b, R, T, tau);
-  // b > 64: sixteen waves of eight columns (109 VGPRs, four waves per SIMD
-  // hide more of the column step's latency than eight waves of sixteen)
-  return rows <= 128 ? leaf_launch<16, 8, 2>(c, A, lda, m, L, b, R, T, tau)
-                     : leaf_launch<16, 8, 4>(c, A, lda, m, L, b, R, T, tau);
+  return leaf16(c, A, lda, m, L, rows, b, R, T, tau, nullptr, 0);
 }
 
 int64_t leaf_capacity_rows(int64_t b) {
