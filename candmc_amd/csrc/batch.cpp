@@ -34,7 +34,7 @@ struct Group {
   BatchProb* d_bp = nullptr;     // the device table (d_seg follows it)
   BatchSeg* d_seg = nullptr;
   // byte offsets into the batch arena
-  size_t leafR, leafT, leafTau, nodeR, nodeV2, nodeT, nodeTau, C, Y, W, Uinv, Winv, LinvT, cnt, qflags, bytes;
+  size_t leafR, leafT, leafTau, nodeR, nodeV2, nodeT, nodeTau, C, Y, W, Uinv, cnt, qflags, bytes;
 };
 
 }  // namespace
@@ -177,8 +177,6 @@ int plan_group(cqr_ctx* c, cqr_batch* bt, Group& g, bool alloc = true) {
   g.Y = s.add(8 * (size_t)g.total_rows * b);
   g.W = s.add(8 * np * bb);
   g.Uinv = s.add(8 * np * bb);
-  g.Winv = s.add(8 * np * bb);
-  g.LinvT = s.add(8 * np * bb);
   g.cnt = s.add(8 * CQR_TREE_FLAGS * nn);
   g.qflags = s.add(8 * nn * (size_t)((b + 15) / 16));
   g.bytes = s.bytes;
@@ -210,12 +208,11 @@ int ensure_batch_ws(cqr_ctx* c, cqr_batch* bt) {
   return CQR_OK;
 }
 
-// The six launches of one group on the context's stream.
+// The launches of one group on the context's stream.
 int run_group(cqr_ctx* c, cqr_batch* bt, const Group& g, double* A, double* Tt) {
   char* base = static_cast<char*>(bt->ws);
   auto at = [&](size_t o) { return reinterpret_cast<double*>(base + o); };
   const int b = g.b, np = (int)g.probs.size();
-  const int64_t bb = (int64_t)b * b;
   uint64_t* cnt = reinterpret_cast<uint64_t*>(base + g.cnt);
   uint64_t* qf = reinterpret_cast<uint64_t*>(base + g.qflags);
   CQR_TRY(fill_u64(c, cnt, CQR_TREE_FLAGS * (int64_t)std::max(g.total_nodes, 1)));
@@ -226,14 +223,10 @@ int run_group(cqr_ctx* c, cqr_batch* bt, const Group& g, double* A, double* Tt) 
                                g.total_nodes, b, g.d_bp, g.d_seg, g.nseg_tree));
   CQR_TRY(launch_q1_batched(c, at(g.nodeV2), at(g.nodeT), at(g.leafT), A, at(g.C), at(g.Y), qf, g.total_items, b,
                             g.d_bp, g.d_seg + g.nseg_tree, g.nseg_q1));
-  CQR_TRY(hr_core_batched(c, g.d_bp, np, at(g.Y), at(g.leafR), at(g.nodeR), A, at(g.W), at(g.Uinv), at(g.Winv),
-                          at(g.LinvT), b));
+  // LU of every Q1 top, [L\S·R], W, U⁻¹ and Tᵀ_p = −L_p⁻¹·W_pᵀ   (W = −T·Y1ᵀ)
+  CQR_TRY(hr_core_batched(c, g.d_bp, np, at(g.Y), at(g.leafR), at(g.nodeR), A, at(g.W), at(g.Uinv), Tt, b));
   // A_p(b:, :) = Q1_p(b:, :)·U_p⁻¹   (hh_recon.cxx:294-301)
-  CQR_TRY(update_y_batched(c, g.d_bp, g.d_seg + g.nseg_tree + g.nseg_q1, g.nseg_y, g.ytiles, b, at(g.Y),
-                           at(g.Uinv), A));
-  // Tᵀ_p = −L_p⁻¹·W_pᵀ   (W = −T·Y1ᵀ)
-  return gemm_f64_batched_prob(c, 1, 1, b, b, b, -1.0, bmat(at(g.LinvT), b, bb), SM_UNIT_UPPER, bmat(at(g.W), b, bb),
-                               SM_UPPER, 0.0, bmat(Tt, b, 0, BM_PROB_T), SM_NONE, np, g.d_bp, 0, 0, b);
+  return update_y_batched(c, g.d_bp, g.d_seg + g.nseg_tree + g.nseg_q1, g.nseg_y, g.ytiles, b, at(g.Y), at(g.Uinv), A);
 }
 
 int run_all(cqr_ctx* c, cqr_batch* bt, double* A, double* Tt) {

@@ -158,11 +158,7 @@ int make_plan(int64_t m, int64_t b, int64_t nleaves_hint, int64_t leaf_rows,
 //   BM_LEAFROWS_SHIFTED p + rowoff(z+zoff)  (the sender's rows of tree pair z)
 // m < 0 or k < 0 stands for the rows of leaf z.
 // ---------------------------------------------------------------------------
-//   BM_PROB_Y   p + bp[z].yoff + prow, ld bp[z].m   (problem z's Q1 block)
-//   BM_PROB_A   p + bp[z].aoff + prow, ld bp[z].m   (problem z's A block)
-//   BM_PROB_T   p + bp[z].toff                     (problem z's Tᵀ block)
-enum { BM_STRIDED = 0, BM_LEAFROWS = 1, BM_SHIFTED = 2, BM_PROB_Y = 3, BM_PROB_A = 4, BM_PROB_T = 5,
-       BM_LEAFROWS_SHIFTED = 6 };
+enum { BM_STRIDED = 0, BM_LEAFROWS = 1, BM_SHIFTED = 2, BM_LEAFROWS_SHIFTED = 3 };
 struct BMat {
   const double* p;
   int64_t ld;
@@ -264,12 +260,10 @@ int q1_items_per_problem(int L, int b);
 int batched_y_tile_rows();
 int update_y_batched(cqr_ctx* c, const BatchProb* bp, const BatchSeg* seg, int nseg, int total_tiles, int b,
                      const double* Y, const double* Uinv, double* A);
+// Householder reconstruction of every problem of a group (hr_kernel.hip): W
+// and U⁻¹ b×b per problem, Tᵀ at the problem's toff.
 int hr_core_batched(cqr_ctx* c, const BatchProb* bp, int nprob, const double* Y, const double* leafR,
-                    const double* nodeR, double* Abase, double* W, double* Uinv, double* Winv, double* LinvT, int b);
-int gemm_f64_batched_prob(cqr_ctx* c, int ta, int tb, int m, int n, int k, double alpha, const BMat& A, int smA,
-                          const BMat& B, int smB, double beta, const BMat& C, int smC, int nprob, const BatchProb* bp,
-                          int64_t prow, int m_prob, int max_m);
-
+                    const double* nodeR, double* Abase, double* W, double* Uinv, double* Tt, int b);
 // Leaves of 64 < b ≤ 128 columns and at most 256 rows (ptree_kernel.hip)
 int leaf16(cqr_ctx* c, double* A, int64_t lda, int64_t m, int L, int64_t rows, int b, double* R, double* T, double* tau,
            const BatchProb* bp, int nprob);
@@ -280,12 +274,24 @@ int leaf_qr(cqr_ctx* c, double* A, int64_t lda, int64_t m, int L, int b, double*
 int tree_level(cqr_ctx* c, double* Rleaf, int n, int node0, int b, double* V2, double* T,
                double* tau);
 int bgemm(cqr_ctx* c, const BgemmArgs& g, int batch, int max_m);
-// With Tt (b = 128 only): also Tᵀ, and U⁻¹·Tᵀ into M2 when non-null, and the
-// top b rows of the explicit Y and of Y·Tᵀ into Ye / YT (ld ldy) when non-null.
-int hr_core(cqr_ctx* c, const double* Q1top, int64_t ldq, const double* Rroot, double* Atop,
-            int64_t lda, double* W, double* Uinv, double* Winv, double* LinvT, int64_t* signs, int b,
-            double* Tt = nullptr, double* M2 = nullptr, double* Ye = nullptr, double* YT = nullptr,
-            int64_t ldy = 0);
+// Householder reconstruction of a panel's top block (hr_kernel.hip, b ≤ 128):
+// signed LU of Q1top − S; Atop := [L \\ S·R], W = U·S, U⁻¹ (ld b, zeros below
+// the diagonal), and whichever of the others are non-null: the signs, Tᵀ, T,
+// T⁻ᵀ (all ld b, zeros outside their triangle), M2 = U⁻¹·Tᵀ (needs Tt), and
+// the top b rows of the explicit Y and of Y·Tᵀ (ld ldy).
+struct HrCore {
+  const double* Q1top;
+  int64_t ldq;
+  const double* Rroot;
+  double* Atop;
+  int64_t lda;
+  double *W, *Uinv;
+  int b;
+  int64_t* signs = nullptr;
+  double *Tt = nullptr, *T = nullptr, *invTT = nullptr, *M2 = nullptr, *Ye = nullptr, *YT = nullptr;
+  int64_t ldy = 0;
+};
+int hr_core(cqr_ctx* c, const HrCore& a);
 int launch_diag(cqr_ctx* c, const double* T, int64_t ldt, double* tau, int b);
 int launch_signed_nlu(cqr_ctx* c, double* A, int64_t lda, double* R, int64_t lda_R,
                       int64_t* signs, int b);
@@ -422,8 +428,6 @@ struct LsqRun {
 int lstsq_refine(cqr_ctx* c, const double* A, int64_t lda, int64_t m, int64_t n, const double* B, int64_t ldb,
                  int64_t nr, double* X, int64_t ldx, int64_t b, const double* Af, int64_t ldf, const double* Tt,
                  int prec, int max_iter, double tol, bool escalate, char* base, const LsqWS& w, LsqRun& out);
-int hh_recon_core(cqr_ctx* c, double* A, int64_t lda, int64_t m, int64_t b, double* W,
-                  double* T, double* invT_T, double* Tt, int64_t nleaves);
 // Looks up the device address of the fixed scratch array of noalloc.hip
 // (device current); cqr_create calls it once per context.
 int noalloc_setup(cqr_ctx* c);

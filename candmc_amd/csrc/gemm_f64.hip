@@ -7,8 +7,8 @@
 // One kernel template serves all three: 128×128 block tile, 4 waves of
 // 64×64, v_mfma_f64_16x16x4f64, LDS double buffering with a register
 // prefetch of the next K slab.  The ROLE template argument only tags the
-// instantiation (0 general, 1 Z = Yᵀ·A, 2 A −= Y·Z', 3 batched per-leaf
-// products) so that kernel traces attribute time to each use.
+// instantiation (0 general, 1 Z = Yᵀ·A, 2 A −= Y·Z') so that kernel traces
+// attribute time to each use.
 #include "cqr_device.h"
 #include "cqr_internal.h"
 
@@ -31,34 +31,7 @@ struct GemmArgs {
   int64_t ldc;
   int64_t kchunk;        // rows of K per split (grid.z splits)
   int64_t split_stride;  // > 0: write raw partial sums to C + z·split_stride
-  // batched form (grid.z = batch index, no split): per-z operand addresses
-  int batched;
-  int a_mode, b_mode, c_mode;  // BM_STRIDED / BM_LEAFROWS / BM_SHIFTED
-  int64_t a_zs, b_zs, c_zs;
-  int64_t pm;                  // panel rows for BM_LEAFROWS
-  int pL, zoff;
-  int m_leaf;                  // m = rows of leaf z
-  int smC;                     // SM_UPPER: store zeros below the diagonal
-  // batched by problem (BM_PROB_*): per-z addresses and sizes from a table
-  const BatchProb* bp;
-  int64_t prow;                // row shift inside the problem's block
-  int m_prob;                  // m = rows of problem z − prow
 };
-
-__device__ __forceinline__ int64_t leaf_row0(int64_t z, int64_t m, int64_t L) { return (z * m) / L; }
-
-__device__ __forceinline__ const double* zaddr(const double* p, int mode, int64_t zs, int z, const GemmArgs& g) {
-  if (mode == BM_LEAFROWS) return p + leaf_row0(z, g.pm, g.pL);
-  if (mode == BM_SHIFTED) return p + (int64_t)(z + g.zoff) * zs;
-  if (mode == BM_PROB_Y) return p + g.bp[z].yoff + g.prow;
-  if (mode == BM_PROB_A) return p + g.bp[z].aoff + g.prow;
-  if (mode == BM_PROB_T) return p + g.bp[z].toff;
-  return p + (int64_t)z * zs;
-}
-// leading dimension of a per-problem operand (its block is m×·, ld m)
-__device__ __forceinline__ int64_t zld(int64_t ld, int mode, int z, const GemmArgs& g) {
-  return (mode == BM_PROB_Y || mode == BM_PROB_A) ? g.bp[z].m : ld;
-}
 
 __device__ __forceinline__ double gmask(double v, int64_t r, int64_t c, int sm) {
   switch (sm) {
@@ -124,23 +97,8 @@ __global__ void __launch_bounds__(256) mfma_gemm_f64(GemmArgs g) {
   double* C = g.C;
   int64_t Mrows = g.m, kbeg, kend;
   int64_t lda = g.lda, ldb = g.ldb, ldc = g.ldc;
-  if (g.batched) {
-    const int z = blockIdx.z;
-    A = zaddr(g.A, g.a_mode, g.a_zs, z, g);
-    B = zaddr(g.B, g.b_mode, g.b_zs, z, g);
-    C = const_cast<double*>(zaddr(g.C, g.c_mode, g.c_zs, z, g));
-    lda = zld(lda, g.a_mode, z, g);
-    ldb = zld(ldb, g.b_mode, z, g);
-    ldc = zld(ldc, g.c_mode, z, g);
-    if (g.m_leaf) Mrows = leaf_row0(z + 1, g.pm, g.pL) - leaf_row0(z, g.pm, g.pL);
-    if (g.m_prob) Mrows = g.bp[z].m - g.prow;
-    kbeg = 0;
-    kend = g.k;
-    if (m0 >= Mrows) return;   // whole block out of this batch entry's rows
-  } else {
-    kbeg = (int64_t)blockIdx.z * g.kchunk;
-    kend = min(g.k, kbeg + g.kchunk);
-  }
+  kbeg = (int64_t)blockIdx.z * g.kchunk;
+  kend = min(g.k, kbeg + g.kchunk);
   const bool full_mn = (m0 + BM <= Mrows) && (n0 + BN <= g.n);
 
   // Each thread loads 8 elements of the A slab and 8 of the B slab:
@@ -292,7 +250,6 @@ __global__ void __launch_bounds__(256) mfma_gemm_f64(GemmArgs g) {
         if (!row_ok || !(full_mn || gn < g.n)) continue;
         double val = alpha * (double)acc[i][j][v];
         if (has_beta) val += g.beta * cold[4 * j + v];
-        if (g.smC == SM_UPPER && gm > gn) val = 0.0;
         C[gm + gn * ldc] = val;
       }
   }
@@ -379,7 +336,6 @@ static void launch_kind(cqr_ctx* c, int ta, int tb, dim3 grid, const GemmArgs& g
   }
   if (kind == PK_GEMM_YTA) launch_role<1>(c->stream, ta, tb, grid, g);
   else if (kind == PK_GEMM_UPD) launch_role<2>(c->stream, ta, tb, grid, g);
-  else if (kind == PK_BGEMM) launch_role<3>(c->stream, ta, tb, grid, g);
   else launch_role<0>(c->stream, ta, tb, grid, g);
 }
 
@@ -574,27 +530,6 @@ static int gemm_f64_impl(cqr_ctx* c, int ta, int tb, int64_t m, int64_t n, int64
   g.C = scratch; g.ldc = m; g.kchunk = kc; g.split_stride = m * n;
   CQR_TRY(launch_mfma(c, ta, tb, g, ns, kind, prec));
   return launch_splitk_reduce(c, scratch, m * n, ns, m, n, C, ldc, alpha, beta);
-}
-
-// Batched over the problems of a group: operand modes BM_PROB_* and
-// BM_STRIDED; m_prob selects per-problem rows (m of problem z − prow).
-int gemm_f64_batched_prob(cqr_ctx* c, int ta, int tb, int m, int n, int k, double alpha, const BMat& A, int smA,
-                          const BMat& B, int smB, double beta, const BMat& C, int smC, int nprob, const BatchProb* bp,
-                          int64_t prow, int m_prob, int max_m) {
-  if (nprob <= 0 || n <= 0 || max_m <= 0) return CQR_OK;
-  GemmArgs g{};
-  g.m = m_prob ? max_m : m; g.n = n; g.k = k; g.alpha = alpha; g.beta = beta;
-  g.A = A.p; g.lda = A.ld; g.smA = smA; g.B = B.p; g.ldb = B.ld; g.smB = smB; g.C = const_cast<double*>(C.p);
-  g.ldc = C.ld; g.kchunk = k; g.split_stride = 0;
-  g.batched = 1;
-  g.a_mode = A.mode; g.b_mode = B.mode; g.c_mode = C.mode;
-  g.a_zs = A.zs; g.b_zs = B.zs; g.c_zs = C.zs;
-  g.smC = smC; g.bp = bp; g.prow = prow; g.m_prob = m_prob;
-  dim3 grid((unsigned)((max_m + 127) / 128), (unsigned)((n + 127) / 128), (unsigned)nprob);
-  hipEvent_t ev = prof_begin(c);
-  launch_kind(c, ta, tb, grid, g, PK_GEMM_SMALL);
-  prof_end(c, ev, PK_GEMM_SMALL, 0.0, 0.0);
-  return check_launch(c, "mfma_gemm_f64_batched_prob");
 }
 
 size_t gemm_f64_scratch_doubles(int64_t m, int64_t n, int64_t k) {

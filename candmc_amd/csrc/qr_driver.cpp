@@ -15,7 +15,7 @@ int launch_copy2d(cqr_ctx* c, const double* src, int64_t lds, double* dst, int64
 // Panel workspace: every buffer TSQR + HR needs for one m×b panel.
 // ---------------------------------------------------------------------------
 struct PanelWS {
-  size_t leafR, leafT, leafTau, nodeR, nodeV2, nodeT, nodeTau, C, Y, Uinv, Winv, LinvT, signs, Wtmp;
+  size_t leafR, leafT, leafTau, nodeR, nodeV2, nodeT, nodeTau, C, Y, Uinv, Wtmp;
 };
 
 static PanelWS panel_layout(const TsqrPlan& p, Sizer& s) {
@@ -31,9 +31,11 @@ static PanelWS panel_layout(const TsqrPlan& p, Sizer& s) {
   w.C = s.add(8 * L * bb);
   w.Y = s.add(8 * (size_t)p.m * b);
   w.Uinv = s.add(8 * 2 * bb);   // [U⁻¹ | U⁻¹·Tᵀ], b×2b
-  w.Winv = s.add(8 * bb);
-  w.LinvT = s.add(8 * bb);
-  w.signs = s.add(8 * b);
+  // spare: the size stays what callers' footprints and the row limit of the
+  // fixed scratch (noalloc.hip) were set by
+  s.add(8 * bb);
+  s.add(8 * bb);
+  s.add(8 * b);
   w.Wtmp = s.add(8 * bb);
   return w;
 }
@@ -83,39 +85,26 @@ int hh_recon_panel(cqr_ctx* c, double* A, int64_t lda, int64_t m, int64_t b, dou
   if (c->gate_at) CQR_HIP(c, hipEventRecord(c->ev_gate, c->stream));
   // K4: LU(Q1_top − S), R := S·R, W = U·S (hh_recon.cxx:282-308)
   double* Wd = W ? W : at(w.Wtmp);
-  int64_t* sg = signs_out ? signs_out : reinterpret_cast<int64_t*>(base + w.signs);
   double* Uinv = at(w.Uinv);
   const bool expl = m > b && Tt && Ye && YT;
-  // at b = 128 the HR core also forms Tᵀ (and, for the explicit Y, U⁻¹·Tᵀ
-  // and the top b rows of Y and Y·Tᵀ) in the same launch
-  const bool fused = Tt && b == 128;
-  CQR_TRY(hr_core(c, Y, m, Rroot, A, lda, Wd, Uinv, at(w.Winv), at(w.LinvT), sg, bi, fused ? Tt : nullptr,
-                  fused && expl ? Uinv + bb : nullptr, fused && expl ? Ye : nullptr, fused && expl ? YT : nullptr,
-                  m));
-  // T = −W·L⁻ᵀ, Tᵀ = −L⁻¹·Wᵀ, T⁻ᵀ = −W⁻ᵀ·L (W = −T·Y1ᵀ)
-  if (Tt && !fused)
-    CQR_TRY(gemm_f64_ws(c, 1, 1, b, b, b, -1.0, at(w.LinvT), b, SM_UNIT_UPPER, Wd, b, SM_UPPER, 0.0, Tt, b,
-                        nullptr));
+  // ... and in the same launch T = −W·L⁻ᵀ, Tᵀ, T⁻ᵀ = −W⁻ᵀ·L (W = −T·Y1ᵀ) and,
+  // for the explicit Y, U⁻¹·Tᵀ and the top b rows of Y and of Y·Tᵀ
+  HrCore h{};
+  h.Q1top = Y; h.ldq = m; h.Rroot = Rroot; h.Atop = A; h.lda = lda; h.W = Wd; h.Uinv = Uinv; h.b = bi;
+  h.signs = signs_out; h.Tt = Tt; h.T = T; h.invTT = invT_T;
+  if (expl) {
+    h.M2 = Uinv + bb;
+    h.Ye = Ye; h.YT = YT; h.ldy = m;
+  }
+  CQR_TRY(hr_core(c, h));
   // Y = Q1·U⁻¹ below the top b rows (hh_recon.cxx:294-301)
   // (U⁻¹ is stored with explicit zeros below its diagonal: a plain GEMM)
   if (expl) {
-    if (!fused) {
-      CQR_TRY(gemm_f64_ws(c, 0, 0, b, b, b, 1.0, Uinv, b, SM_NONE, Tt, b, SM_NONE, 0.0, Uinv + bb, b, nullptr));
-      CQR_TRY(launch_copy_unit_lower(c, A, lda, Ye, m, b, b));
-      // Y1·Tᵀ = −Wᵀ exactly (W = −T·Y1ᵀ); formed as a product like the rest
-      CQR_TRY(gemm_f64_ws(c, 0, 0, b, b, b, 1.0, A, lda, SM_UNIT_LOWER, Tt, b, SM_NONE, 0.0, YT, m, nullptr));
-    }
     CQR_TRY(update_gemm_split(c, m - b, 2 * b, b, b, Y + b, m, Uinv, b, A + b, lda, Ye + b, m, YT + b, m,
                               PK_GEMM_SMALL));
   } else if (m > b) {
     CQR_TRY(update_gemm(c, m - b, b, b, 1.0, Y + b, m, Uinv, b, 0.0, A + b, lda, PK_GEMM_SMALL, 0));
   }
-  if (T)
-    CQR_TRY(gemm_f64_ws(c, 0, 0, b, b, b, -1.0, Wd, b, SM_UPPER, at(w.LinvT), b, SM_UNIT_UPPER, 0.0, T, b,
-                        nullptr));
-  if (invT_T)
-    CQR_TRY(gemm_f64_ws(c, 1, 0, b, b, b, -1.0, at(w.Winv), b, SM_UPPER, A, lda, SM_UNIT_LOWER, 0.0, invT_T, b,
-                        nullptr));
   return CQR_OK;
 }
 

@@ -3,7 +3,6 @@
 //   tree_node     K2  QR of stacked triangles [R_top; R_bot] (dtpqrt l=b)
 //   bgemm         small batched GEMMs for the reverse tree, the per-leaf
 //                 block-reflector products and the Y formation
-//   hr_core       K4  LU without pivoting of Q1_top − S, W, U⁻¹, L⁻ᵀ
 // plus element-wise helpers.  Leaves are contiguous row blocks
 // [floor(l·m/L), floor((l+1)·m/L)); the tree pairs receiver r with sender
 // r + ceil(n/2) on a level of n live ranks (alg/QR/tsqr/bitree_tsqr.cxx:172-208),
@@ -329,327 +328,6 @@ __global__ void __launch_bounds__(256) bgemm_kernel(BgemmArgs g) {
   }
 }
 
-// ---------------------------------------------------------------------------
-// Signed LU of a b×b block (alg/QR/hh_recon/hh_recon.cxx:43-70), b ≤ 128,
-// 512 threads, in LDS (M, ld b).  Step i picks s_i (−1 if the pivot is
-// positive, else +1), subtracts it from the pivot, scales the column below
-// the pivot by its reciprocal (|pivot| ≥ 1) and updates the later columns.
-// Blocked by eight: one wave factors the block's columns from registers
-// (pivot-row entries by readlane, no barrier); one thread per later column
-// solves its eight block rows with the unit-lower diagonal block (U12);
-// the rank-8 update of the trailing matrix runs as FP64 MFMA tiles over all
-// waves.  On exit M holds L\U and sgn the signs.
-// ---------------------------------------------------------------------------
-__device__ __forceinline__ void signed_lu_lds(const double* __restrict__ src, int64_t ld, double* M, int ldm, double* sgn, int b) {
-  constexpr int NT = 512, NB = 8, RPL = 2;
-  const int tid = threadIdx.x, lane = tid & 63, w = wave_id();
-  {
-    // all 32 loads of a thread in flight at once (clamped addresses, then masked stores)
-    double v[16][2];
-#pragma unroll
-    for (int j = 0; j < 16; ++j)
-#pragma unroll
-      for (int s = 0; s < 2; ++s) {
-        const int cc = w + 8 * j, rr = lane + 64 * s;
-        v[j][s] = src[(cc < b && rr < b) ? rr + (int64_t)cc * ld : 0];
-      }
-#pragma unroll
-    for (int j = 0; j < 16; ++j)
-#pragma unroll
-      for (int s = 0; s < 2; ++s) {
-        const int cc = w + 8 * j, rr = lane + 64 * s;
-        if (cc < b && rr < b) M[rr + cc * ldm] = v[j][s];
-      }
-  }
-  __syncthreads();
-  for (int c0 = 0; c0 < b; c0 += NB) {
-    const int nb = min(NB, b - c0);
-    if (w == 0) {
-      double pn[RPL][NB];
-#pragma unroll
-      for (int s = 0; s < RPL; ++s) {
-        const int row = lane + 64 * s;
-#pragma unroll
-        for (int j = 0; j < NB; ++j) pn[s][j] = (row >= c0 && row < b && j < nb) ? M[row + (c0 + j) * ldm] : 0.0;
-      }
-#pragma unroll
-      for (int jj = 0; jj < NB; ++jj) {
-        if (jj < nb) {
-        const int i = c0 + jj, hi = i >> 6, pl = i & 63;
-        const double pv = readlane_d(hi ? pn[1][jj] : pn[0][jj], pl);
-        const double sg = pv > 0.0 ? -1.0 : 1.0;
-        const double piv = pv - sg;
-        const double rp = 1.0 / piv;
-#pragma unroll
-        for (int s = 0; s < RPL; ++s) {
-          const int row = lane + 64 * s;
-          if (row > i) pn[s][jj] *= rp;
-          if (row == i) pn[s][jj] = piv;
-        }
-        if (lane == 0) sgn[i] = sg;
-#pragma unroll
-        for (int j2 = jj + 1; j2 < NB; ++j2) {
-          if (j2 < nb) {
-            const double u = readlane_d(hi ? pn[1][j2] : pn[0][j2], pl);
-#pragma unroll
-            for (int s = 0; s < RPL; ++s)
-              if (lane + 64 * s > i) pn[s][j2] -= pn[s][jj] * u;
-          }
-        }
-        }
-      }
-#pragma unroll
-      for (int s = 0; s < RPL; ++s) {
-        const int row = lane + 64 * s;
-#pragma unroll
-        for (int j = 0; j < NB; ++j)
-          if (row >= c0 && row < b && j < nb) M[row + (c0 + j) * ldm] = pn[s][j];
-      }
-    }
-    __syncthreads();
-    const int j0 = c0 + nb;
-    if (j0 >= b) break;
-    // U12 = L11⁻¹·A12, one thread per later column
-    for (int j = j0 + tid; j < b; j += NT) {
-      double u[NB];
-#pragma unroll
-      for (int jj = 0; jj < NB; ++jj) u[jj] = jj < nb ? M[c0 + jj + j * ldm] : 0.0;
-#pragma unroll
-      for (int jj = 1; jj < NB; ++jj)
-#pragma unroll
-        for (int p = 0; p < jj; ++p)
-          if (jj < nb) u[jj] -= M[c0 + jj + (c0 + p) * ldm] * u[p];
-#pragma unroll
-      for (int jj = 1; jj < NB; ++jj)
-        if (jj < nb) M[c0 + jj + j * ldm] = u[jj];
-    }
-    __syncthreads();
-    // A22 −= L21·U12 on 16×16 MFMA tiles (K = 8)
-    const int nt = (b - j0 + 15) / 16;
-    auto tile = [&](int t) {
-      const int r0 = j0 + 16 * (t % nt), q0 = j0 + 16 * (t / nt);
-      auto x = [&](int m, int k) {
-        const int r = r0 + m;
-        const bool ok = r < b && k < nb;
-        return ok ? M[r + (c0 + k) * ldm] : 0.0;
-      };
-      auto y = [&](int k, int n) {
-        const int q = q0 + n;
-        const bool ok = q < b && k < nb;
-        return ok ? M[c0 + k + q * ldm] : 0.0;
-      };
-      const dbl4 acc = mfma_tile16(x, y, 0, NB, lane);
-      const int r = r0 + (lane & 15);
-#pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const int q = q0 + (lane >> 4) + 4 * v;
-        if (r < b && q < b) M[r + q * ldm] -= acc[v];
-      }
-    };
-    // two tiles per wave in flight
-    for (int t = w; t < nt * nt; t += 2 * NT / 64) {
-      tile(t);
-      if (t + NT / 64 < nt * nt) tile(t + NT / 64);
-    }
-    __syncthreads();
-  }
-  __syncthreads();
-}
-
-// K4: Householder reconstruction core (one workgroup).  M is kept in LDS
-// with leading dimension b + 1.
-__device__ __forceinline__ void hr_core_body(const double* __restrict__ Q1top, int64_t ldq, const double* __restrict__ Rroot,
-                             double* __restrict__ Atop, int64_t lda, double* __restrict__ W,
-                             double* __restrict__ Uinv, double* __restrict__ Winv, double* __restrict__ LinvT,
-                             int64_t* __restrict__ signs, int b) {
-  constexpr int NT = 512;
-  extern __shared__ double smem[];
-  const int ldm = b + 1;
-  double* M = smem;            // b×b, ld b+1
-  double* sgn = M + b * ldm;   // b
-  double* d = sgn + b;         // b
-  const int tid = threadIdx.x, lane = tid & 63, w = wave_id();
-  signed_lu_lds(Q1top, ldq, M, ldm, sgn, b);
-  // outputs: L below the diagonal of Atop, S·R on and above it, W = U·S
-  {
-    double rv[16][2];
-#pragma unroll
-    for (int j = 0; j < 16; ++j)
-#pragma unroll
-      for (int s = 0; s < 2; ++s) {
-        const int cc = w + 8 * j, rr = lane + 64 * s;
-        rv[j][s] = Rroot[(cc < b && rr < b) ? rr + cc * b : 0];
-      }
-#pragma unroll
-    for (int j = 0; j < 16; ++j)
-#pragma unroll
-      for (int s = 0; s < 2; ++s) {
-        const int cc = w + 8 * j, rr = lane + 64 * s;
-        if (cc < b && rr < b) {
-          const double mv = M[rr + cc * ldm];
-          Atop[rr + cc * lda] = rr > cc ? mv : sgn[rr] * rv[j][s];
-          W[rr + cc * b] = rr <= cc ? mv * sgn[cc] : 0.0;
-        }
-      }
-  }
-  if (signs)
-    for (int p = tid; p < b; p += NT) signs[p] = (int64_t)sgn[p];
-  for (int p = tid; p < b; p += NT) d[p] = 1.0 / M[p + p * ldm];
-  __syncthreads();
-  tri_inv_upper_lds<NT>(M, ldm, d, b);
-  FOR_RC(rr, cc, b, NT) {
-    const double u = rr <= cc ? M[rr + cc * ldm] : 0.0;
-    Uinv[rr + cc * b] = u;
-    Winv[rr + cc * b] = sgn[rr] * u;        // W⁻¹ = S·U⁻¹
-  }
-  __syncthreads();
-  // L⁻ᵀ: load Lᵀ (unit upper) from Atop and invert
-  {
-    double lv[16][2];
-#pragma unroll
-    for (int j = 0; j < 16; ++j)
-#pragma unroll
-      for (int s = 0; s < 2; ++s) {
-        const int cc = w + 8 * j, rr = lane + 64 * s;
-        lv[j][s] = Atop[(cc < b && rr < cc) ? cc + rr * lda : 0];
-      }
-#pragma unroll
-    for (int j = 0; j < 16; ++j)
-#pragma unroll
-      for (int s = 0; s < 2; ++s) {
-        const int cc = w + 8 * j, rr = lane + 64 * s;
-        if (cc < b && rr < b) M[rr + cc * ldm] = rr < cc ? lv[j][s] : 0.0;
-      }
-  }
-  for (int p = tid; p < b; p += NT) d[p] = 1.0;
-  __syncthreads();
-  tri_inv_upper_lds<NT>(M, ldm, d, b);
-  FOR_RC(rr, cc, b, NT) LinvT[rr + cc * b] = rr <= cc ? M[rr + cc * ldm] : 0.0;
-}
-
-// The products that follow the HR core in a QR_2D panel, in the same
-// workgroup (b = 128, 8 waves; wave w owns the 16-row block w of each
-// result).  On entry L⁻ᵀ is in M (upper part, ld b+1) and W, U⁻¹, L are in
-// global memory, stored by this workgroup.
-//   Tt = Tᵀ = −L⁻¹·Wᵀ  (lower; T = −W·L⁻ᵀ, hh_recon.cxx:282-308)
-//   M2 = U⁻¹·Tᵀ        (so that Q1·[U⁻¹ | M2] gives Y and Y·Tᵀ at once)
-//   with Ye: Ye top = [unit lower L],  YT top = Y1·Tᵀ = −Wᵀ  (W = −T·Y1ᵀ)
-__device__ __forceinline__ void hr_tail_body(double* __restrict__ M, int ldm, const double* __restrict__ Atop,
-                                             int64_t lda, const double* __restrict__ W,
-                                             const double* __restrict__ Uinv, double* __restrict__ Tt,
-                                             double* __restrict__ M2, double* __restrict__ Ye,
-                                             double* __restrict__ YT, int64_t ldy) {
-  constexpr int b = 128;
-  const int tid = threadIdx.x, lane = tid & 63, w = wave_id();
-  const int r16 = lane & 15, q4 = lane >> 4;
-  const int i0 = 16 * w;
-  __syncthreads();   // W, U⁻¹ and L stored by every wave are visible
-  dbl4 tt[8];
-#pragma unroll
-  for (int tn = 0; tn < 8; ++tn) {
-    tt[tn] = dbl4{0.0, 0.0, 0.0, 0.0};
-    if (tn > w) continue;   // Tᵀ is lower: tiles right of the diagonal are zero
-    // L⁻¹[i][k] = L⁻ᵀ[k][i], nonzero for k ≤ i;  Wᵀ[k][j] = W[j][k], nonzero for j ≤ k
-    auto x = [&](int m, int k) {
-      const int i = i0 + m;
-      const bool ok = k <= i;
-      const double v = M[ok ? k + i * ldm : 0];   // clamped, loaded unconditionally
-      return ok ? v : 0.0;
-    };
-    auto y = [&](int k, int n) {
-      const int j = 16 * tn + n;
-      const bool ok = j <= k && k < b;
-      const double v = W[ok ? j + k * b : 0];
-      return ok ? v : 0.0;
-    };
-    tt[tn] = mfma_tile16_acc4(x, y, 16 * tn, i0 + 16, lane);
-  }
-  __syncthreads();   // every wave is done reading L⁻ᵀ from M
-  // Tᵀ (negated) into M, column-major ld ldm, and out
-#pragma unroll
-  for (int tn = 0; tn < 8; ++tn)
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      const int i = i0 + r16, j = 16 * tn + q4 + 4 * v;
-      const double val = -tt[tn][v];
-      M[i + j * ldm] = val;
-      Tt[i + j * b] = val;
-    }
-  __syncthreads();
-  if (M2) {
-#pragma unroll
-    for (int tn = 0; tn < 8; ++tn) {
-      // U⁻¹[i][k] nonzero for k ≥ i; Tᵀ[k][j] nonzero for k ≥ j
-      auto x = [&](int m, int k) {
-        const int i = i0 + m;
-        const bool ok = k >= i && k < b;
-        const double v = Uinv[ok ? i + k * b : 0];
-        return ok ? v : 0.0;
-      };
-      auto y = [&](int k, int n) {
-        const int j = 16 * tn + n;
-        const bool ok = k >= j && k < b;
-        const double v = M[ok ? k + j * ldm : 0];
-        return ok ? v : 0.0;
-      };
-      const dbl4 acc = mfma_tile16_acc4(x, y, max(i0, 16 * tn), b, lane);
-#pragma unroll
-      for (int v = 0; v < 4; ++v) M2[(i0 + r16) + (16 * tn + q4 + 4 * v) * b] = acc[v];
-    }
-  }
-  if (Ye) {
-    FOR_RC(rr, cc, b, 512) {
-      Ye[rr + cc * ldy] = rr > cc ? Atop[rr + cc * lda] : (rr == cc ? 1.0 : 0.0);
-      YT[rr + cc * ldy] = rr >= cc ? -W[cc + rr * b] : 0.0;
-    }
-  }
-}
-
-__global__ void __launch_bounds__(512)
-hr_core_kernel(const double* __restrict__ Q1top, int64_t ldq, const double* __restrict__ Rroot,
-               double* __restrict__ Atop, int64_t lda, double* __restrict__ W,
-               double* __restrict__ Uinv, double* __restrict__ Winv, double* __restrict__ LinvT,
-               int64_t* __restrict__ signs, int b, double* __restrict__ Tt, double* __restrict__ M2,
-               double* __restrict__ Ye, double* __restrict__ YT, int64_t ldy) {
-  hr_core_body(Q1top, ldq, Rroot, Atop, lda, W, Uinv, Winv, LinvT, signs, b);
-  if (Tt) {
-    extern __shared__ double smem[];
-    hr_tail_body(smem, b + 1, Atop, lda, W, Uinv, Tt, M2, Ye, YT, ldy);
-  }
-}
-
-// Batched: workgroup p handles problem p (its Q1 top in Y, its root R).
-__global__ void __launch_bounds__(512)
-hr_core_batched_kernel(const BatchProb* __restrict__ bp, const double* __restrict__ Y,
-                       const double* __restrict__ leafR, const double* __restrict__ nodeR,
-                       double* __restrict__ Abase, double* __restrict__ W, double* __restrict__ Uinv,
-                       double* __restrict__ Winv, double* __restrict__ LinvT, int b) {
-  const BatchProb P = bp[blockIdx.x];
-  const int64_t bb = (int64_t)b * b, p = blockIdx.x;
-  const double* Rroot = P.L > 1 ? nodeR + (int64_t)(P.node0 + P.L - 2) * bb : leafR + (int64_t)P.leaf0 * bb;
-  hr_core_body(Y + P.yoff, P.m, Rroot, Abase + P.aoff, P.m, W + p * bb, Uinv + p * bb, Winv + p * bb,
-               LinvT + p * bb, nullptr, b);
-}
-
-// a5 standalone: signed LU of a b×b block with R scaling.
-__global__ void __launch_bounds__(512)
-signed_nlu_kernel(double* __restrict__ A, int64_t lda, double* __restrict__ R, int64_t ldr,
-                  int64_t* __restrict__ signs, int b) {
-  constexpr int NT = 512;
-  extern __shared__ double smem[];
-  const int ldm = b + 1;
-  double* M = smem;
-  double* sgn = M + b * ldm;
-  const int tid = threadIdx.x;
-  signed_lu_lds(A, lda, M, ldm, sgn, b);
-  FOR_RC(rr, cc, b, NT) {
-    A[rr + cc * lda] = M[rr + cc * ldm];
-    if (R && rr <= cc && sgn[rr] < 0) R[rr + cc * ldr] = -R[rr + cc * ldr];
-  }
-  if (signs)
-    for (int p = tid; p < b; p += NT) signs[p] = (int64_t)sgn[p];
-}
-
 // Inverse of a triangular b×b matrix (one workgroup).  upper: invert the
 // upper triangle of X; else the lower triangle (through its transpose).
 __device__ __forceinline__ void tri_inverse_body(const double* __restrict__ X, int64_t ldx, double* __restrict__ Xi,
@@ -875,39 +553,6 @@ int bgemm(cqr_ctx* c, const BgemmArgs& g, int batch, int max_m) {
 }
 
 static int big_lds_attr(cqr_ctx* c, const void* k) { return set_max_lds(c, k, 163840); }
-
-int hr_core(cqr_ctx* c, const double* Q1top, int64_t ldq, const double* Rroot, double* Atop,
-            int64_t lda, double* W, double* Uinv, double* Winv, double* LinvT, int64_t* signs, int b,
-            double* Tt, double* M2, double* Ye, double* YT, int64_t ldy) {
-  if (Tt && b != 128) return set_err(c, CQR_ERR_UNSUPPORTED, "hr_core: fused Tt needs b = 128");
-  if (Ye && !(Tt && YT)) return set_err(c, CQR_ERR_INVALID, "hr_core: Ye needs Tt and YT");
-  CQR_TRY(big_lds_attr(c, (const void*)hr_core_kernel));
-  const size_t lds = sizeof(double) * ((size_t)b * (b + 1) + 2 * b);
-  hipEvent_t ev = prof_begin(c);
-  hipLaunchKernelGGL(hr_core_kernel, dim3(1), dim3(512), lds, c->stream, Q1top, ldq, Rroot, Atop,
-                     lda, W, Uinv, Winv, LinvT, signs, b, Tt, M2, Ye, YT, ldy);
-  const double bbb = (double)b * b * b;
-  prof_end(c, ev, PK_HR, (2.0 / 3.0) * bbb + (Tt ? bbb / 3.0 : 0.0) + (M2 ? bbb : 0.0), 64.0 * b * b);
-  return check_launch(c, "hr_core");
-}
-
-int hr_core_batched(cqr_ctx* c, const BatchProb* bp, int nprob, const double* Y, const double* leafR,
-                    const double* nodeR, double* Abase, double* W, double* Uinv, double* Winv, double* LinvT, int b) {
-  CQR_TRY(big_lds_attr(c, (const void*)hr_core_batched_kernel));
-  const size_t lds = sizeof(double) * ((size_t)b * (b + 1) + 2 * b);
-  hipEvent_t ev = prof_begin(c);
-  hipLaunchKernelGGL(hr_core_batched_kernel, dim3(nprob), dim3(512), lds, c->stream, bp, Y, leafR, nodeR, Abase, W,
-                     Uinv, Winv, LinvT, b);
-  prof_end(c, ev, PK_HR, nprob * (2.0 / 3.0) * b * (double)b * b, nprob * 64.0 * b * b);
-  return check_launch(c, "hr_core_batched");
-}
-
-int launch_signed_nlu(cqr_ctx* c, double* A, int64_t lda, double* R, int64_t lda_R, int64_t* signs, int b) {
-  CQR_TRY(big_lds_attr(c, (const void*)signed_nlu_kernel));
-  const size_t lds = sizeof(double) * ((size_t)b * (b + 1) + b);
-  hipLaunchKernelGGL(signed_nlu_kernel, dim3(1), dim3(512), lds, c->stream, A, lda, R, lda_R, signs, b);
-  return check_launch(c, "signed_nlu");
-}
 
 int launch_tri_inverse(cqr_ctx* c, const double* X, int64_t ldx, double* Xi, int64_t ldi, int b,
                        int upper, int unit) {
