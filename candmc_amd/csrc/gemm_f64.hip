@@ -561,10 +561,8 @@ size_t wy_update_ws_doubles(int64_t m, int64_t n, int b) {
   return gemm_f64_scratch_doubles(b, n, m) + 2 * (size_t)b * n + 64;
 }
 
-int lean_gemm(cqr_ctx* c, int ak, int64_t M, int64_t N, int64_t K, double alpha, const double* A, int64_t lda,
-              const double* B, int64_t ldb, double beta, double* C, int64_t ldc, double* scratch, int nsplit,
-              int kind, int* used);
-
+int lean_gemm(cqr_ctx* c, int64_t M, int64_t N, int64_t K, const double* A, int64_t lda, const double* B, int64_t ldb,
+              double* scratch, int cap, int kind, int* used);
 
 // FP64 update with the unmasked bulk on the lean kernel: rows [0, bt) of Y
 // (its unit-lower top block) go through the masked general kernel, rows
@@ -582,8 +580,7 @@ static int wy_update_f64_split(cqr_ctx* c, const double* Y, int64_t ldy, int smY
   CQR_TRY(launch_mfma(c, 1, 0, g, 1, PK_GEMM_YTA));
   // slots 1..: Y(bt:m)ᵀ·A(bt:m) on the lean kernel
   int used = 0;
-  CQR_TRY(lean_gemm(c, 1, b, n, m - bt, 1.0, Y + bt, ldy, A + bt, lda, 0.0, nullptr, 0, part + (int64_t)b * n,
-                    ns - 1, PK_GEMM_YTA, &used));
+  CQR_TRY(lean_gemm(c, b, n, m - bt, Y + bt, ldy, A + bt, lda, part + (int64_t)b * n, ns - 1, PK_GEMM_YTA, &used));
   const int nslots = 1 + used;
   CQR_TRY(launch_splitk_reduce(c, part, (int64_t)b * n, nslots, b, n, Z, b, 1.0, 0.0));
   CQR_TRY(gemm_f64_impl(c, t_trans ? 1 : 0, 0, b, n, b, 1.0, Tt, b, SM_LOWER, Z, b, SM_NONE, 0.0, Zp, b, nullptr));
@@ -641,7 +638,7 @@ int wy_explicit_yta(cqr_ctx* c, const double* Ye, int64_t m, int64_t n, int b, c
   const int ns = np ? (int)(np / ((size_t)b * n)) : 0;
   if (ns >= 2) {
     int used = 0;
-    CQR_TRY(lean_gemm(c, 1, b, n, m, 1.0, Ye, m, A, lda, 0.0, nullptr, 0, part, ns, PK_GEMM_YTA, &used));
+    CQR_TRY(lean_gemm(c, b, n, m, Ye, m, A, lda, part, ns, PK_GEMM_YTA, &used));
     return launch_splitk_reduce(c, part, (int64_t)b * n, used, b, n, Z, b, 1.0, 0.0);
   }
   return gemm_f64_impl(c, 1, 0, b, n, m, 1.0, Ye, m, SM_NONE, A, lda, SM_NONE, 0.0, Z, b, np ? part : nullptr,
