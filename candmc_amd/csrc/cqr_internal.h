@@ -268,6 +268,14 @@ int hr_core_batched(cqr_ctx* c, const BatchProb* bp, int nprob, const double* Y,
 int leaf16(cqr_ctx* c, double* A, int64_t lda, int64_t m, int L, int64_t rows, int b, double* R, double* T, double* tau,
            const BatchProb* bp, int nprob);
 
+// The implicit TSQR Q applied leaf by leaf and level by level with B in
+// registers (apply16_kernel.hip), for plans and column counts it takes.
+bool apply16_takes(const TsqrPlan& p, int64_t k);
+int apply16_leaves(cqr_ctx* c, int trans, const TsqrPlan& p, const double* Y, int64_t ldy, const double* leafT, double* B,
+                   int64_t ldb, int64_t k);
+int apply16_level(cqr_ctx* c, int trans, const TsqrPlan& p, int lv, const double* nodeV2, const double* nodeT, double* B,
+                  int64_t ldb, int64_t k);
+
 // Kernel launchers (tsqr_kernels.hip)
 int leaf_qr(cqr_ctx* c, double* A, int64_t lda, int64_t m, int L, int b, double* R, double* T,
             double* tau);

@@ -14,8 +14,10 @@
 //   Qᵀ·B: the leaves (B_l −= V_l·T_lᵀ·(V_lᵀ·B_l)), then the levels forward:
 //           X = Tᵀ·(B_z + V2ᵀ·B_s);  B_z −= X;  B_s −= V2·X
 //   Q·B:  the levels backward with T in place of Tᵀ, then the leaves with T_l.
-// Every step is one batched GEMM launch over all leaves or over one level's
-// pairs (bgemm, addressing leaves by their row offsets); B is processed in
+// The leaves and each level are one launch that keeps B's columns in registers
+// (apply16_kernel.hip) while a leaf has at most 512 rows; beyond (b ≤ 32 only)
+// every step is one batched GEMM launch over all leaves or over one level's
+// pairs (bgemm, addressing leaves by their row offsets) and B is processed in
 // column chunks that bound the scratch to 2·L·b·kc doubles.
 #include "cqr_device.h"
 #include "cqr_internal.h"
@@ -183,8 +185,14 @@ int apply_level(cqr_ctx* c, int trans, const TsqrPlan& p, int lv, const double* 
 // apply_scratch_bytes(p, k) bytes.
 int tsqr_apply(cqr_ctx* c, int trans, const TsqrPlan& p, const double* Y, int64_t ldy, const double* leafT,
                const double* nodeV2, const double* nodeT, double* B, int64_t ldb, int64_t k, double* scratch) {
-  const int64_t kc = chunk_cols(p, k);
   const int nlv = (int)p.levels.size();
+  if (apply16_takes(p, k)) {
+    if (trans) CQR_TRY(apply16_leaves(c, 1, p, Y, ldy, leafT, B, ldb, k));
+    for (int i = 0; i < nlv; ++i) CQR_TRY(apply16_level(c, trans, p, trans ? i : nlv - 1 - i, nodeV2, nodeT, B, ldb, k));
+    if (!trans) CQR_TRY(apply16_leaves(c, 0, p, Y, ldy, leafT, B, ldb, k));
+    return CQR_OK;
+  }
+  const int64_t kc = chunk_cols(p, k);
   double* W = scratch;
   double* W2 = scratch + p.nleaves * p.b * kc;
   for (int64_t j0 = 0; j0 < k; j0 += kc) {
