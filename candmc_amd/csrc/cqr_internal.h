@@ -37,7 +37,7 @@ struct cqr_ctx {
   int* d_flag = nullptr;        // device flag for non-finite scans / tree timeouts
   uint64_t* d_cnt = nullptr;    // progress words: tree nodes, then (second half) leaves
   int* d_terr = nullptr;        // set by a tree node whose wait for a child timed out
-  uint64_t* d_qflags = nullptr; // per (node, column block) flags of construct_Q1
+  uint64_t* d_qflags = nullptr; // per (node, strip pair) flags of construct_Q1
   uint64_t* d_sflags = nullptr; // per 128-row block flags of the one-launch triangular solve
   double* h_pin = nullptr;      // 64 doubles of pinned host memory for small device-to-host reads
   hipEvent_t ev_host = nullptr; // recorded after a copy into h_pin
