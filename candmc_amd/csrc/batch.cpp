@@ -11,6 +11,8 @@
 // cqr_batch_tune picks by timing the candidates on the caller's data.
 #include <algorithm>
 #include <cstring>
+#include <functional>
+#include <list>
 #include <vector>
 
 #include "cqr_internal.h"
@@ -431,6 +433,7 @@ struct LsqBatchPlan {
   size_t oA = 0, oT = 0, oBp = 0, oG = 0, oR = 0, bytes = 0;
   std::vector<size_t> bp_off;     // per group, inside oBp
   size_t refine = 0;
+  std::list<std::vector<LsqProb>> tabs;   // on their way to the device until the call's last sync
 };
 
 int plan_lsq_batch(cqr_ctx* c, int64_t np, const cqr_request* rq, LsqBatchPlan& P) {
@@ -484,6 +487,88 @@ int plan_lsq_batch(cqr_ctx* c, int64_t np, const cqr_request* rq, LsqBatchPlan& 
   return CQR_OK;
 }
 
+// No request's X overlaps anything else of the batch: the requests can then
+// advance together.
+bool outputs_apart(int64_t np, const cqr_request* rq) {
+  struct Span {
+    const double *lo, *hi;
+    bool out;
+  };
+  std::vector<Span> v;
+  v.reserve(3 * np);
+  for (int64_t p = 0; p < np; ++p) {
+    const cqr_request& r = rq[p];
+    v.push_back(Span{r.A, r.A + (r.n - 1) * r.lda + r.m, false});
+    v.push_back(Span{r.B, r.B + (r.nrhs - 1) * r.ldb + r.m, false});
+    v.push_back(Span{r.X, r.X + (r.nrhs - 1) * r.ldx + r.n, true});
+  }
+  std::sort(v.begin(), v.end(), [](const Span& a, const Span& b) { return std::less<const double*>()(a.lo, b.lo); });
+  const double *any = nullptr, *out = nullptr;   // the furthest ends so far
+  for (const Span& x : v) {
+    if (std::less<const double*>()(x.lo, x.out ? any : out)) return false;
+    any = std::max(any, x.hi, std::less<const double*>());
+    if (x.out) out = std::max(out, x.hi, std::less<const double*>());
+  }
+  return true;
+}
+
+// Consecutive requests whose tables, states and partial sums fit the arena
+// that the factorization's buffers and the single refinement share (one
+// request always does).
+struct LsqChunk {
+  int64_t p0, p1;
+  int nslab, nmax;
+  LsqProb* probs;
+  LsqState* states;
+};
+int run_chunks(cqr_ctx* c, LsqBatchPlan& P, int64_t np, const cqr_request* rq, char* base, bool parts,
+               const std::function<int(const LsqChunk&)>& run) {
+  const cqr_batch& bt = P.bt;
+  const size_t room = P.bytes - P.oG;
+  char* at = base + P.oG;
+  for (int64_t p0 = 0, p1; p0 < np; p0 = p1) {
+    P.tabs.emplace_back();
+    std::vector<LsqProb>& tab = P.tabs.back();
+    size_t used = 0;
+    int nslab = 0, nmax = 0;
+    for (p1 = p0; p1 < np && p1 - p0 < 32768; ++p1) {
+      const cqr_request& r = rq[p1];
+      const int64_t slab = lsq_slab_rows(r.m), ns = (r.m + slab - 1) / slab;
+      const size_t part = parts ? 8 * (size_t)(ns * r.n * r.nrhs) : 0;
+      if (p1 > p0 && used + part + (p1 + 1 - p0) * (sizeof(LsqProb) + sizeof(LsqState)) > room) break;
+      LsqProb q{};
+      q.A = r.A;
+      q.B = r.B;
+      q.X = r.X;
+      q.Y = reinterpret_cast<double*>(base + P.oA) + bt.aoff[p1];
+      q.T = reinterpret_cast<double*>(base + P.oT) + bt.toff[p1];
+      q.part = reinterpret_cast<double*>(at + used);
+      q.lda = r.lda;
+      q.ldb = r.ldb;
+      q.ldx = r.ldx;
+      q.m = r.m;
+      q.slab = slab;
+      q.n = (int)r.n;
+      q.nr = (int)r.nrhs;
+      q.nslab = (int)ns;
+      tab.push_back(q);
+      used += part;
+      nslab = std::max(nslab, q.nslab);
+      nmax = std::max(nmax, q.n);
+    }
+    LsqChunk k;
+    k.p0 = p0;
+    k.p1 = p1;
+    k.nslab = nslab;
+    k.nmax = nmax;
+    k.probs = reinterpret_cast<LsqProb*>(at + used);
+    k.states = reinterpret_cast<LsqState*>(at + used + sizeof(LsqProb) * tab.size());
+    CQR_HIP(c, hipMemcpyAsync(k.probs, tab.data(), sizeof(LsqProb) * tab.size(), hipMemcpyHostToDevice, c->stream));
+    CQR_TRY(run(k));
+  }
+  return CQR_OK;
+}
+
 }  // namespace
 
 size_t cqr_lstsq_batched_workspace_bytes(int64_t nprob, const cqr_request* reqs) {
@@ -519,22 +604,64 @@ int cqr_lstsq_batched(cqr_ctx* c, int64_t nprob, const cqr_request* reqs, int ma
     CQR_HIP(c, hipMemcpyAsync(g.d_bp, g.htab.data(), g.htab.size(), hipMemcpyHostToDevice,
                               c->stream));
   }
-  for (int64_t p = 0; p < nprob; ++p)
-    CQR_TRY(launch_copy2d(c, reqs[p].A, reqs[p].lda, Ap + bt.aoff[p], bt.m[p], bt.m[p], bt.n[p]));
+  const bool apart = outputs_apart(nprob, reqs);
+  if (apart) {
+    CQR_TRY(run_chunks(c, P, nprob, reqs, base, false, [&](const LsqChunk& k) {
+      return launch_lsq_copy(c, k.probs, (int)(k.p1 - k.p0), k.nslab);
+    }));
+  } else {
+    for (int64_t p = 0; p < nprob; ++p)
+      CQR_TRY(launch_copy2d(c, reqs[p].A, reqs[p].lda, Ap + bt.aoff[p], bt.m[p], bt.m[p], bt.n[p]));
+  }
   int rc = CQR_OK;
   for (Group& g : bt.groups)
     if ((rc = run_group(c, &bt, g, Ap, Tp)) != CQR_OK) break;
-  for (int64_t p = 0; p < nprob; ++p) {
+  auto alone = [&](int64_t p) {
     const cqr_request& r = reqs[p];
     LsqRun run;
     LsqWS w;
     refine_ws(r.m, r.n, r.nrhs, r.n, &w);
-    status[p] = rc != CQR_OK ? rc
-                             : lstsq_refine(c, r.A, r.lda, r.m, r.n, r.B, r.ldb, r.nrhs, r.X, r.ldx, r.n,
-                                            Ap + bt.aoff[p], r.m, Tp + bt.toff[p], CQR_PREC_F64, max_iter, tol, false,
-                                            base + P.oR, w, run);
+    status[p] = lstsq_refine(c, r.A, r.lda, r.m, r.n, r.B, r.ldb, r.nrhs, r.X, r.ldx, r.n, Ap + bt.aoff[p], r.m,
+                             Tp + bt.toff[p], CQR_PREC_F64, max_iter, tol, false, base + P.oR, w, run);
     if (iters) iters[p] = run.iters;
     if (last_update) last_update[p] = run.rel;
+  };
+  if (rc != CQR_OK) {
+    for (int64_t p = 0; p < nprob; ++p) {
+      status[p] = rc;
+      if (iters) iters[p] = 0;
+      if (last_update) last_update[p] = 0.0;
+    }
+  } else if (apart) {
+    std::vector<LsqState> st;
+    CQR_TRY(run_chunks(c, P, nprob, reqs, base, true, [&](const LsqChunk& k) {
+      const int np = (int)(k.p1 - k.p0);
+      st.resize(np);
+      CQR_TRY(launch_lsq_solve(c, k.probs, k.states, np, k.nslab, k.nmax, 0, tol));
+      // two steps between looks at the states: most requests need no third
+      for (int it = 1;; it += 2) {
+        for (int i = it; i < it + 2 && i <= max_iter; ++i)
+          CQR_TRY(launch_lsq_solve(c, k.probs, k.states, np, k.nslab, k.nmax, i, tol));
+        CQR_HIP(c, hipMemcpyAsync(st.data(), k.states, sizeof(LsqState) * np, hipMemcpyDeviceToHost, c->stream));
+        CQR_HIP(c, hipStreamSynchronize(c->stream));
+        bool active = false;
+        for (const LsqState& x : st) active |= x.state == LSQ_ACTIVE;
+        if (!active || it + 2 > max_iter) break;
+      }
+      for (int64_t p = k.p0; p < k.p1; ++p) {
+        const LsqState& x = st[p - k.p0];
+        if (x.state == LSQ_DONE || (max_iter == 0 && x.state == LSQ_ACTIVE)) {
+          status[p] = CQR_OK;
+          if (iters) iters[p] = x.iters;
+          if (last_update) last_update[p] = x.rel;
+        } else {
+          alone(p);
+        }
+      }
+      return (int)CQR_OK;
+    }));
+  } else {
+    for (int64_t p = 0; p < nprob; ++p) alone(p);
   }
   for (Group& g : bt.groups) g.d_bp = nullptr;   // arena memory, not owned
   bt.ws = nullptr;

@@ -436,6 +436,27 @@ struct LsqRun {
 int lstsq_refine(cqr_ctx* c, const double* A, int64_t lda, int64_t m, int64_t n, const double* B, int64_t ldb,
                  int64_t nr, double* X, int64_t ldx, int64_t b, const double* Af, int64_t ldf, const double* Tt,
                  int prec, int max_iter, double tol, bool escalate, char* base, const LsqWS& w, LsqRun& out);
+// Solve and refinement of many one-panel requests in a few launches
+// (lsq_batch.hip): request p's factors in Y (ld m) and T (Tᵀ, ld n), `part`
+// for nslab·n·nr partial sums.
+struct LsqProb {
+  const double *A, *B, *T;
+  double *Y, *X, *part;
+  int64_t lda, ldb, ldx, m, slab;
+  int n, nr, nslab;
+};
+// LSQ_LEFT: R is not finite or the steps stopped contracting; lstsq_refine
+// takes the request from its factors.
+enum { LSQ_ACTIVE = 0, LSQ_DONE = 1, LSQ_LEFT = 2 };
+struct LsqState {
+  int state, iters;
+  double rel;      // the last step taken, relative to the solution
+};
+int64_t lsq_slab_rows(int64_t m);
+int launch_lsq_copy(cqr_ctx* c, const LsqProb* probs, int np, int nslab);
+// it = 0: the first solution; it ≥ 1: one refinement step.  nslab, nmax: the
+// most slabs and columns of a request.
+int launch_lsq_solve(cqr_ctx* c, const LsqProb* probs, LsqState* states, int np, int nslab, int nmax, int it, double tol);
 // Looks up the device address of the fixed scratch array of noalloc.hip
 // (device current); cqr_create calls it once per context.
 int noalloc_setup(cqr_ctx* c);
