@@ -22,7 +22,6 @@
 // the leaves and 0.23 ms in the first level.
 #include "cqr_device.h"
 #include "cqr_internal.h"
-#include "leaf_body.h"
 #include "panel16.h"
 
 namespace cqr {
@@ -30,32 +29,6 @@ namespace cqr {
 namespace {
 
 constexpr int W = 4;   // waves, and strips of 16 columns, of a workgroup
-
-typedef double dbl2a __attribute__((ext_vector_type(2), aligned(8)));
-
-// Four rows p[0..3] of a column, of which `left` exist.
-__device__ __forceinline__ dbl4 rows4_load(const double* p, int left, bool ok) {
-  if (ok && left >= 4) {
-    const dbl2a lo = *reinterpret_cast<const dbl2a*>(p), hi = *reinterpret_cast<const dbl2a*>(p + 2);
-    return dbl4{lo[0], lo[1], hi[0], hi[1]};
-  }
-  dbl4 x = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-  for (int v = 0; v < 4; ++v)
-    if (ok && v < left) x[v] = p[v];
-  return x;
-}
-__device__ __forceinline__ void rows4_store(double* p, const dbl4& x, int left, bool ok) {
-  if (!ok) return;
-  if (left >= 4) {
-    *reinterpret_cast<dbl2a*>(p) = dbl2a{x[0], x[1]};
-    *reinterpret_cast<dbl2a*>(p + 2) = dbl2a{x[2], x[3]};
-  } else {
-#pragma unroll
-    for (int v = 0; v < 4; ++v)
-      if (v < left) p[v] = x[v];
-  }
-}
 
 // acc + Σ V_tᵀ·a_t, and a_t += V_t·u, over the groups of four tiles that meet
 // [lo, hi); tiles of such a group outside it are zero in V.
@@ -148,7 +121,7 @@ apply_leaf16_kernel(const double* __restrict__ Y, int64_t ldy, const double* __r
 #pragma unroll
     for (int i = 0; i < TPW; ++i) {
       const int t = w + W * i, row = 16 * t + 4 * g;
-      pv[i] = rows4_load(p + row, r - row, t >= kk && cc < b);
+      pv[i] = p16_rows_load(p + row, r - row, t >= kk && cc < b);
       if (t == kk)
 #pragma unroll
         for (int v = 0; v < 4; ++v) pv[i][v] = 4 * g + v > c ? pv[i][v] : (4 * g + v == c && cc < b ? 1.0 : 0.0);
@@ -165,7 +138,7 @@ apply_leaf16_kernel(const double* __restrict__ Y, int64_t ldy, const double* __r
   fetch(panel(0));
   dbl4 a[RT];
 #pragma unroll
-  for (int t = 0; t < RT; ++t) a[t] = rows4_load(Bc + 16 * t, r - 16 * t - 4 * g, ok);
+  for (int t = 0; t < RT; ++t) a[t] = p16_rows_load(Bc + 16 * t, r - 16 * t - 4 * g, ok);
   put(0);
   for (int s = 0; s < nblk; ++s) {
     const int kk = panel(s), buf = s & 1;
@@ -180,7 +153,7 @@ apply_leaf16_kernel(const double* __restrict__ Y, int64_t ldy, const double* __r
   }
 #pragma unroll
   for (int t = 0; t < RT; ++t)
-    if (16 * t < r) rows4_store(Bc + 16 * t, a[t], r - 16 * t - 4 * g, ok);
+    if (16 * t < r) p16_rows_store(Bc + 16 * t, a[t], r - 16 * t - 4 * g, ok);
 }
 
 // One tree level: workgroup (pair, 16·W columns); the pair's receiver is leaf
@@ -212,7 +185,7 @@ apply_node16_kernel(const double* __restrict__ nodeV2, const double* __restrict_
 #pragma unroll
     for (int i = 0; i < TPW; ++i) {
       const int t = w + W * i, row = 16 * t + 4 * g;
-      pv[i] = rows4_load(p + row, b - row, t <= kk && cc < b);
+      pv[i] = p16_rows_load(p + row, b - row, t <= kk && cc < b);
       if (t == kk)
 #pragma unroll
         for (int v = 0; v < 4; ++v) pv[i][v] = 4 * g + v <= c ? pv[i][v] : 0.0;
@@ -235,7 +208,7 @@ apply_node16_kernel(const double* __restrict__ nodeV2, const double* __restrict_
   fetch(panel(0));
   dbl4 a[N];
 #pragma unroll
-  for (int t = 0; t < N; ++t) a[t] = rows4_load(Bs + 16 * t, b - 16 * t - 4 * g, ok);
+  for (int t = 0; t < N; ++t) a[t] = p16_rows_load(Bs + 16 * t, b - 16 * t - 4 * g, ok);
   put(0);
   for (int s = 0; s < nblk; ++s) {
     const int kk = panel(s), buf = s & 1;
@@ -257,7 +230,7 @@ apply_node16_kernel(const double* __restrict__ nodeV2, const double* __restrict_
   }
 #pragma unroll
   for (int t = 0; t < N; ++t)
-    if (16 * t < b) rows4_store(Bs + 16 * t, a[t], b - 16 * t - 4 * g, ok);
+    if (16 * t < b) p16_rows_store(Bs + 16 * t, a[t], b - 16 * t - 4 * g, ok);
 }
 
 template <int RT>

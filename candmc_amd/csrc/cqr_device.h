@@ -100,6 +100,9 @@ __device__ inline double xreduce(double (&v)[N], int lane) {
   return xr_cross_rows(s);
 }
 
+// First row of leaf l of L.
+__device__ __forceinline__ int64_t leaf_off(int64_t l, int64_t m, int64_t L) { return (l * m) / L; }
+
 // ---------------------------------------------------------------------------
 // Hand-off of data between workgroups of one launch without cache-wide
 // fences.  Every value that crosses workgroups is written and read with
@@ -203,19 +206,6 @@ __device__ inline double recip_nr(double x) {
   r = fma(r, e, r);
   e = fma(-x, r, 1.0);
   return fma(r, e, r);
-}
-
-// dlarfg when no rescaling can be needed (ss = ‖x‖² in (2^-960, 2^960),
-// |alpha| < 2^480): |beta| = sqrt(alpha² + ss) ≥ 2^-480, so knt = 0; the
-// two quotients use recip_nr.  Returns false (h untouched) otherwise.
-__device__ inline bool dlarfg_fast(double alpha, double ss, Reflector& h) {
-  if (!(ss > 0x1p-960 && ss < 0x1p960) || !(fabs(alpha) < 0x1p480)) return false;
-  const double beta = -copysign(sqrt(fma(alpha, alpha, ss)), alpha);
-  h.beta = beta;
-  h.tau = (beta - alpha) * recip_nr(beta);
-  h.scal = recip_nr(alpha - beta);
-  h.knt = 0;
-  return true;
 }
 
 // Robust norm finish: `ss` is the plain sum of squares; when it may have

@@ -36,6 +36,32 @@ __device__ __forceinline__ void p16_store(double* __restrict__ X, const dbl4& y,
   for (int v = 0; v < 4; ++v) xp[4 * v * P16_LD] = y[v];
 }
 
+typedef double dbl2a __attribute__((ext_vector_type(2), aligned(8)));
+
+// Four rows p[0..3] of a column, of which `left` exist.
+__device__ __forceinline__ dbl4 p16_rows_load(const double* p, int left, bool ok) {
+  if (ok && left >= 4) {
+    const dbl2a lo = *reinterpret_cast<const dbl2a*>(p), hi = *reinterpret_cast<const dbl2a*>(p + 2);
+    return dbl4{lo[0], lo[1], hi[0], hi[1]};
+  }
+  dbl4 x = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+  for (int v = 0; v < 4; ++v)
+    if (ok && v < left) x[v] = p[v];
+  return x;
+}
+__device__ __forceinline__ void p16_rows_store(double* p, const dbl4& x, int left, bool ok) {
+  if (!ok) return;
+  if (left >= 4) {
+    *reinterpret_cast<dbl2a*>(p) = dbl2a{x[0], x[1]};
+    *reinterpret_cast<dbl2a*>(p + 2) = dbl2a{x[2], x[3]};
+  } else {
+#pragma unroll
+    for (int v = 0; v < 4; ++v)
+      if (v < left) p[v] = x[v];
+  }
+}
+
 // s[v] += x_t[v](column J)·x_t[v] over four tiles.  The leading s_nop covers
 // the two wait states a DPP source needs after a VALU write.
 template <int J>
@@ -169,14 +195,29 @@ __device__ __forceinline__ void p16_larfg(double alpha, double ss, double& beta,
 // the end the panel's compact-WY T, transposed; Vs (RT tiles), where the
 // strip is kept for the slow path and the scaled vectors are left; Ds (one
 // tile), the pivot tile before and after.
-template <int RT, bool NODE>
+// With PARTS > 1 a leaf's panel is spread over as many waves, `part` of them
+// this one, all with RT tiles and one more, the pivot tile in part 0 and an
+// ordinary one in the others (its values then live in pr[0..3]; Ds is its
+// place in Vs).  Each part publishes its share of a column's dot products in
+// `ex` (two buffers of PARTS + 1 rows of sixteen, the last one the pivot row),
+// and after a workgroup barrier all of them form the same reflector.
+template <int RT, bool NODE, int PARTS = 1>
 struct Panel16 {
-  // the tiles [H, RT) are skipped as a whole once they are zero
-  static constexpr int H = RT > 8 ? 8 : RT > 4 ? 4 : RT;
+  double* ex;
+  int part = 0;
+  // the tiles [H, RT) are skipped as a whole once they are zero (never in a
+  // tall leaf, whose parts stay full)
+  static constexpr int H = PARTS > 1 ? RT : RT > 8 ? 8 : RT > 4 ? 4 : RT;
   double pr[P16];          // pivot rows
   double tau, scale;
   double ssv, alv, smax;   // what decides the fast range: ‖x‖², alpha per column, largest |dot|
 
+  // part ≠ 0, opaque as nact in column()
+  __device__ __forceinline__ bool low() const {
+    int p = part;
+    asm volatile("" : "+s"(p));
+    return p != 0;
+  }
   // tile row that holds matrix row q of the pivot tile
   __device__ static constexpr int trow_of(int q) { return NODE ? q : (q >> 2) + 4 * (q & 3); }
 
@@ -212,14 +253,27 @@ struct Panel16 {
     if constexpr (RT > H)
       if (__builtin_expect(nact > H, 1)) dots<J, H, RT>(s4, a);
     double s = (s4[0] + s4[1]) + (s4[2] + s4[3]);
-    if constexpr (!NODE) {
+    if (PARTS > 1 && low()) {
+      p16_dotrows<J, 4>(d2, pr);
+      s += d2[0] + d2[1];
+    } else if constexpr (!NODE) {
 #pragma unroll
       for (int q = 0; q + 4 <= N; q += 4) p16_dotrows<J, 4>(d2, pr + J + 1 + q);
       if constexpr (N % 4 != 0) p16_dotrows<J, N % 4>(d2, pr + P16 - N % 4);
     }
     s = xr_cross_rows(s);
-    if constexpr (!NODE) s += d2[0] + d2[1];
-    const double p = pr[J];
+    if constexpr (!NODE) s += PARTS > 1 && low() ? 0.0 : d2[0] + d2[1];
+    double p = pr[J];
+    if constexpr (PARTS > 1) {
+      double* E = ex + (J & 1) * (P16 * (PARTS + 1)) + c;
+      E[P16 * part] = s;                        // four lanes, one value
+      if (!low()) E[P16 * PARTS] = p;
+      __syncthreads();
+      s = E[0];
+#pragma unroll
+      for (int q = 1; q < PARTS; ++q) s += E[P16 * q];
+      p = E[P16 * PARTS];
+    }
     const double ss = readlane_d(s, J), alpha = readlane_d(p, J);
     double beta, tj, scal, rb;
     p16_larfg(alpha, ss, beta, tj, scal, rb);
@@ -229,13 +283,17 @@ struct Panel16 {
     asm volatile("" : "+s"(nact));
     if constexpr (RT > H)
       if (__builtin_expect(nact > H, 1)) axpys<J, H, RT>(a, f);
-    if constexpr (!NODE) {
+    if (PARTS > 1 && low()) {
+      p16_axpyrows<J, 4>(pr, f);
+    } else {
+      if constexpr (!NODE) {
 #pragma unroll
-      for (int q = 0; q + 4 <= N; q += 4) p16_axpyrows<J, 4>(pr + J + 1 + q, f);
-      if constexpr (N % 4 != 0) p16_axpyrows<J, N % 4>(pr + P16 - N % 4, f);
+        for (int q = 0; q + 4 <= N; q += 4) p16_axpyrows<J, 4>(pr + J + 1 + q, f);
+        if constexpr (N % 4 != 0) p16_axpyrows<J, N % 4>(pr + P16 - N % 4, f);
+      }
+      pr[J] = c > J ? fma(-tj, wv, p) : (c == J ? beta : p);
+      Zc[J * P16_LD] = wv * scale * -tj;        // four lanes, one value
     }
-    pr[J] = c > J ? fma(-tj, wv, p) : (c == J ? beta : p);
-    Zc[J * P16_LD] = wv * scale * -tj;          // four lanes, one value
     smax = fmax(smax, fabs(s));
     ssv = c == J ? s : ssv;
     alv = c == J ? p : alv;
@@ -356,7 +414,10 @@ struct Panel16 {
     double* Zc = Zs + c;
 #pragma unroll
     for (int q = 0; q < P16; ++q) pr[q] = Ds[trow_of(q) * P16_LD + c];
-    if (nb < P16)
+    if (PARTS > 1 && part != 0) {
+#pragma unroll
+      for (int v = 0; v < 4; ++v) pr[v] = D[v];
+    } else if (nb < P16)
       for (int q = nb; q < P16; ++q) Zc[q * P16_LD] = 0.0;
 #define P16_STEP(J)                 \
   asm volatile("" : "+s"(nb));      \
@@ -367,11 +428,16 @@ struct Panel16 {
     // the fast range: ‖x‖² in (2^-200, 2^200), |alpha| < 2^200, dots far from
     // overflow; a NaN or infinity fails it
     if (__builtin_amdgcn_ballot_w64(!(ssv > 0x1p-200 && ssv < 0x1p200 && fabs(alv) < 0x1p200 && smax < 0x1p800)) != 0) {
-      slow(Vs, Ds, Zs, nact > H ? RT : H, nb, tau);
+      if (PARTS > 1 && part != 0) return;
+      slow(Vs, Ds, Zs, PARTS > 1 ? RT + 16 * (PARTS - 1) : nact > H ? RT : H, nb, tau);
     } else {
 #pragma unroll
       for (int t = 0; t < RT; ++t)
         if (t < H || nact > H) p16_store(Vs + t * P16_TILE, a[t] * scale, lane);
+      if (PARTS > 1 && part != 0) {
+        p16_store(Ds, dbl4{pr[0], pr[1], pr[2], pr[3]} * scale, lane);
+        return;
+      }
 #pragma unroll
       for (int q = 0; q < P16; ++q) Ds[trow_of(q) * P16_LD + c] = !NODE && q > c ? pr[q] * scale : pr[q];
     }

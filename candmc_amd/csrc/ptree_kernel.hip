@@ -33,7 +33,6 @@
 // problems of up to 16384×128 17.5 → 13.8 ms, QR 32768×4096 43.9 → 38.2 ms.
 #include "cqr_device.h"
 #include "cqr_internal.h"
-#include "leaf_body.h"
 #include "panel16.h"
 
 namespace cqr {
@@ -246,6 +245,183 @@ __device__ __forceinline__ void leaf16_body(double* __restrict__ A, int64_t lda,
 }
 
 // ---------------------------------------------------------------------------
+// A leaf taller than a wave's registers (r ≤ 256·P rows, b ≤ 16·S columns):
+// P waves share a strip, 256 rows each, the first of them with the pivot
+// tile.  They factor a panel together (a barrier a column) and add their shares of each product in LDS (X), so the steps run
+// one after another, with one panel of V in LDS.  Three loops rather than one
+// with roles: the factor() of the strip's own panel then stands in no loop,
+// where its registers spilled.  512×64 leaves take 0.11 ms (0.125 with a
+// reflector at a time over 64-row lanes); hh_recon_qr of 65536×16 234 →
+// 162 µs, ×32 328 → 245, 16384×64 458 → 321 (with the other kernels' gains).
+// ---------------------------------------------------------------------------
+template <int S, int P>
+constexpr int tall_smem_doubles() {
+  return (16 * P + S * (S + 1) / 2 + 1 + (S - 1) * P) * P16_TILE + 2 * P16 * (P + 1);
+}
+
+template <int S, int P>
+__device__ __forceinline__ void leaf16_tall_body(double* __restrict__ A, int64_t lda, int64_t m, int L, int b,
+                                                 double* __restrict__ Rout, double* __restrict__ Tout,
+                                                 double* __restrict__ tauout, const BatchProb* __restrict__ bp,
+                                                 int nprob, int gleaf, double* smem) {
+  constexpr int NB = P16 - 1;
+  int leaf = gleaf;
+  if (bp) {                    // batched: A is the group's base, the problem's block at aoff
+    const BatchProb B = bp[bp_find(bp, nprob, gleaf, BP_LEAF)];
+    A += B.aoff;
+    lda = B.m;
+    m = B.m;
+    L = B.L;
+    leaf = gleaf - B.leaf0;
+  }
+  const int64_t r0 = leaf_off(leaf, m, L);
+  const int r = (int)(leaf_off(leaf + 1, m, L) - r0);
+  const int64_t bb = (int64_t)b * b;
+  double* Rl = Rout + (int64_t)gleaf * bb;
+  double* Tl = Tout + (int64_t)gleaf * bb;
+  double* taul = tauout + (int64_t)gleaf * b;
+  double* Vk = smem;                              // the panel, tile by tile
+  double* Ts = Vk + 16 * P * P16_TILE;            // tiles of T, and one for the pivot tile
+  double* X = Ts + (S * (S + 1) / 2 + 1) * P16_TILE;
+  double* ex = X + (S - 1) * P * P16_TILE;
+
+  const int lane = threadIdx.x & 63, w = wave_id(), strip = w / P, part = w % P;
+  const int c = lane & 15, g = lane >> 4;
+  const int nblk = (b + P16 - 1) / P16;
+  const int col = 16 * strip + c;
+  const bool colok = col < b;
+  const int rg = r - 256 * part - 4 * g;          // rows left from this lane group's first
+  double* Ac = A + r0 + 256 * part + 4 * g + (int64_t)(colok ? col : 0) * lda;
+  const dbl4 zero = {0.0, 0.0, 0.0, 0.0};
+  // loads from clamped rows, then masked: no branch, no mask kept
+  const double* A0 = Ac - 4 * g - 256 * part;     // the leaf's first row
+  auto load = [&](int t) {
+    dbl4 x;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) x[v] = A0[min(256 * part + 4 * g + 16 * t + v, r - 1)];
+#pragma unroll
+    for (int v = 0; v < 4; ++v) x[v] = (colok && 16 * t + v < rg) ? x[v] : 0.0;
+    return x;
+  };
+  dbl4 D = load(0), a[NB];
+#pragma unroll
+  for (int t = 0; t < NB; ++t) {
+    a[t] = load(t + 1);
+    if (t % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+  }
+  if (part == 0 && strip < nblk) {
+    zero_below(Rl, b, strip, lane);
+    zero_below(Tl, b, strip, lane);
+  }
+  double* Vp = Vk + 16 * part * P16_TILE;         // this part's tiles of the panel
+  auto panel = [&](int k) {                       // another strip's panel: its columns, then V and T_kk are there
+    for (int j = 16 * k; j < min(b, 16 * k + 16); ++j) __syncthreads();
+    __syncthreads();
+  };
+  // this part's share of V_kᵀ·(D; a) into X, for all parts after a barrier
+  auto share = [&](int k) {
+    dbl4 top[1] = {D};
+    dbl4 wt = p16_vta<1>(Vp, top, 1, zero, lane);
+    wt = p16_vta<NB>(Vp + P16_TILE, a, NB, wt, lane);
+    p16_store(X + ((strip < k ? strip : strip - 1) * P + part) * P16_TILE, wt, lane);
+  };
+  auto sum = [&](int k) {
+    const double* Xs = X + (strip < k ? strip : strip - 1) * P * P16_TILE;
+    dbl4 wt = p16_load(Xs, lane);
+#pragma unroll
+    for (int q = 1; q < P; ++q) wt += p16_load(Xs + q * P16_TILE, lane);
+    return wt;
+  };
+  // row block k of this strip is final: R(k, strip), and vectors for strip ≤ k
+  auto finish = [&](int k) {
+    if (part != 0) return;
+    if (strip >= k && colok) {
+      const int row = 16 * k + 4 * g;
+#pragma unroll
+      for (int v = 0; v < 4; ++v)
+        if (row + v < b) Rl[row + v + (int64_t)col * b] = row + v <= col ? D[v] : 0.0;
+    }
+    p16_rows_store(Ac + 16 * k, D, rg - 16 * k, colok);
+    D = a[0];
+#pragma unroll
+    for (int t = 0; t + 1 < NB; ++t) a[t] = a[t + 1];
+    a[NB - 1] = zero;
+  };
+  // before its own panel the strip takes the earlier ones in
+  for (int k = 0; k < min(strip, nblk); ++k) {
+    panel(k);
+    if (strip < nblk) share(k);
+    __syncthreads();
+    if (strip < nblk) {
+      const dbl4 u = -p16_xy(Ts + p16_slot(k, k), sum(k), zero, lane);
+      dbl4 top[1] = {D};
+      p16_vu<1>(Vp, top, 1, u, lane);
+      D = top[0];
+      p16_vu<NB>(Vp + P16_TILE, a, NB, u, lane);
+      finish(k);
+    }
+    __syncthreads();
+  }
+  if (strip >= nblk) return;                      // (no barrier is left)
+  {
+    const int k = strip;
+    __builtin_amdgcn_s_setprio(3);
+    Panel16<NB, false, P> F;
+    F.ex = ex;
+    F.part = part;
+    F.factor(D, a, NB, min(P16, b - 16 * k), lane, Ts + p16_slot(k, k), Vp + P16_TILE,
+             part == 0 ? Ts + p16_slot(0, S) : Vp);
+    if (part == 0) {
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const int row = 4 * g + v;
+        Vk[(g + 4 * v) * P16_LD + c] = row > c ? D[v] : (row == c ? 1.0 : 0.0);
+      }
+      if (g == 0 && colok) taul[col] = F.tau;
+    }
+    __builtin_amdgcn_s_setprio(0);
+    __syncthreads();
+    __syncthreads();
+    // the scaled vectors back from LDS
+    if (part == 0) put_t_tile(Tl, b, k, k, p16_load(Ts + p16_slot(k, k), lane), lane);
+    else D = p16_load(Vp, lane);
+#pragma unroll
+    for (int t = 0; t < NB; ++t) a[t] = p16_load(Vp + (t + 1) * P16_TILE, lane);
+    finish(k);
+    __syncthreads();
+  }
+  // after it, the strip's tiles of T
+  dbl4 tnew = zero;
+  for (int k = strip + 1; k < nblk; ++k) {
+    panel(k);
+    share(k);
+    if (part == 0 && strip < k - 2) p16_store(Ts + p16_slot(strip, k - 2), tnew, lane);
+    __syncthreads();
+    if (part == 0) {
+      p16_store(Ts + p16_slot(strip, k), sum(k), lane);
+      if (strip < k - 1) {
+        tnew = p16_tcol(Ts, strip, k - 1, lane);
+        put_t_tile(Tl, b, strip, k - 1, tnew, lane);
+      }
+    }
+    finish(k);
+    __syncthreads();
+  }
+  if (part == 0 && strip < nblk - 1) {
+    if (strip < nblk - 2) p16_store(Ts + p16_slot(strip, nblk - 2), tnew, lane);
+    put_t_tile(Tl, b, strip, nblk - 1, p16_tcol(Ts, strip, nblk - 1, lane), lane);
+  }
+  // the rows below the last panel's block
+  if (strip < nblk) {
+    const int t0 = part == 0 ? nblk : 0;
+    p16_rows_store(Ac + 16 * t0, D, rg - 16 * t0, colok);
+#pragma unroll
+    for (int t = 0; t < NB; ++t)
+      if (t0 + t + 1 < 16) p16_rows_store(Ac + 16 * (t0 + t + 1), a[t], rg - 16 * (t0 + t + 1), colok);
+  }
+}
+
+// ---------------------------------------------------------------------------
 // One tree node per workgroup of W waves (b ≤ 16·W).  The reflectors are
 // [e; v2] with v2 in the bottom triangle: wave w holds the bottom tiles
 // (0..w, w) of its columns and one tile of the top triangle at a time, which
@@ -410,6 +586,14 @@ leaf16_kernel(double* __restrict__ A, int64_t lda, int64_t m, int L, int b, doub
   leaf16_body<W, RT>(A, lda, m, L, b, Rout, Tout, tauout, bp, nprob, blockIdx.x, smem, nullptr, 0);
 }
 
+template <int S, int P>
+__global__ void __launch_bounds__(64 * S * P)
+leaf16_tall_kernel(double* __restrict__ A, int64_t lda, int64_t m, int L, int b, double* __restrict__ Rout,
+                   double* __restrict__ Tout, double* __restrict__ tauout, const BatchProb* __restrict__ bp, int nprob) {
+  extern __shared__ double smem[];
+  leaf16_tall_body<S, P>(A, lda, m, L, b, Rout, Tout, tauout, bp, nprob, blockIdx.x, smem);
+}
+
 // Leaves and tree in one launch (b in (64, 128], leaves of at most 256
 // rows): workgroups [0, L) factor the leaves and announce their R tile by
 // tile, workgroups [L, L + nnodes) are the tree nodes, which start on a
@@ -458,25 +642,34 @@ static int tree_dispatch(cqr_ctx* c, const double* leafR, double* nodeR, double*
   return node16_launch<8>(c, leafR, nodeR, V2, T, tau, cnt, L, nnodes, b, epoch, bp, seg, nseg);
 }
 
-template <int W, int RT>
-static int leaf16_launch(cqr_ctx* c, double* A, int64_t lda, int64_t m, int L, int b, double* R, double* T, double* tau,
-                         const BatchProb* bp, int nprob) {
-  const size_t lds = sizeof(double) * p16_smem_doubles<W, RT>();
-  auto k = leaf16_kernel<W, RT>;
-  CQR_TRY(set_max_lds(c, (const void*)k, (int)lds));
-  hipEvent_t ev = prof_begin(c);
-  hipLaunchKernelGGL(k, dim3(L), dim3(64 * W), lds, c->stream, A, lda, m, L, b, R, T, tau, bp, nprob);
-  prof_end(c, ev, PK_LEAF, 2.0 * m * b * b - (2.0 / 3.0) * L * (double)b * b * b, 16.0 * m * b);
-  return check_launch(c, "leaf16");
-}
-
-// Leaves of 64 < b ≤ 128 columns, rows the largest leaf (≤ 256); with bp the
-// leaves of a batched group.
+// Leaf QR of every row block, rows the largest leaf; with bp the leaves of a
+// batched group.  A wave holds 16 columns of up to 256 rows; taller leaves
+// (b ≤ 64) take two or four waves a strip.
 int leaf16(cqr_ctx* c, double* A, int64_t lda, int64_t m, int L, int64_t rows, int b, double* R, double* T, double* tau,
            const BatchProb* bp, int nprob) {
-  if (b <= 64 || b > 128 || rows > 256) return set_err(c, CQR_ERR_UNSUPPORTED, "leaf16: b = %d, rows = %lld", b, (long long)rows);
-  if (rows <= 128) return leaf16_launch<8, 8>(c, A, lda, m, L, b, R, T, tau, bp, nprob);
-  return leaf16_launch<8, 16>(c, A, lda, m, L, b, R, T, tau, bp, nprob);
+  if (b < 1 || b > 128 || rows > (b <= 32 ? 1024 : b <= 64 ? 512 : 256))
+    return set_err(c, CQR_ERR_UNSUPPORTED, "leaf: b = %d, rows = %lld", b, (long long)rows);
+  auto run = [&](auto k, int waves, int lds_doubles) {
+    const size_t lds = sizeof(double) * lds_doubles;
+    CQR_TRY(set_max_lds(c, (const void*)k, (int)lds));
+    hipEvent_t ev = prof_begin(c);
+    hipLaunchKernelGGL(k, dim3(L), dim3(64 * waves), lds, c->stream, A, lda, m, L, b, R, T, tau, bp, nprob);
+    prof_end(c, ev, PK_LEAF, 2.0 * m * b * b - (2.0 / 3.0) * L * (double)b * b * b, 16.0 * m * b);
+    return check_launch(c, "leaf16");
+  };
+#define CQR_LEAF(W, RT) run(leaf16_kernel<W, RT>, W, p16_smem_doubles<W, RT>())
+#define CQR_TALL(S, P) run(leaf16_tall_kernel<S, P>, S * P, tall_smem_doubles<S, P>())
+  if (rows <= 256) {
+    const bool low = rows <= 128;
+    if (b <= 16) return low ? CQR_LEAF(1, 8) : CQR_LEAF(1, 16);
+    if (b <= 32) return low ? CQR_LEAF(2, 8) : CQR_LEAF(2, 16);
+    if (b <= 64) return low ? CQR_LEAF(4, 8) : CQR_LEAF(4, 16);
+    return low ? CQR_LEAF(8, 8) : CQR_LEAF(8, 16);
+  }
+  if (rows <= 512) return b <= 16 ? CQR_TALL(1, 2) : b <= 32 ? CQR_TALL(2, 2) : CQR_TALL(4, 2);
+  return b <= 16 ? CQR_TALL(1, 4) : CQR_TALL(2, 4);
+#undef CQR_LEAF
+#undef CQR_TALL
 }
 
 template <int RT>

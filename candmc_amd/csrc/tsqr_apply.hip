@@ -21,7 +21,6 @@
 // column chunks that bound the scratch to 2·L·b·kc doubles.
 #include "cqr_device.h"
 #include "cqr_internal.h"
-#include "leaf_body.h"
 
 #include <vector>
 

@@ -1,5 +1,4 @@
 // Panel kernels of the CA-QR hot path for gfx950 (FP64):
-//   leaf_qr       K1  Householder QR of every leaf row block (dgeqrf semantics)
 //   tree_node     K2  QR of stacked triangles [R_top; R_bot] (dtpqrt l=b)
 //   bgemm         small batched GEMMs for the reverse tree, the per-leaf
 //                 block-reflector products and the Y formation
@@ -9,7 +8,6 @@
 // so every address is computed on the device from scalar arguments.
 #include "cqr_device.h"
 #include "cqr_internal.h"
-#include "leaf_body.h"
 
 namespace cqr {
 
@@ -19,19 +17,6 @@ namespace cqr {
 #define FOR_RC(rr, cc, b, NT)                                                     \
   for (int cc = wave_id(); cc < (b); cc += (NT) / 64)                             \
     for (int rr = (int)(threadIdx.x & 63); rr < (b); rr += 64)
-
-// ---------------------------------------------------------------------------
-// K1: leaf QR for b ≤ 64, one workgroup per leaf (body in leaf_body.h; wider
-// panels: leaf16 in ptree_kernel.hip).
-// ---------------------------------------------------------------------------
-template <int WAVES, int CPW, int RPL>
-__global__ void __launch_bounds__(64 * WAVES)
-leaf_qr_kernel(double* __restrict__ A, int64_t lda, int64_t m, int L, int b,
-               double* __restrict__ Rout, double* __restrict__ Tout, double* __restrict__ tauout,
-               const BatchProb* __restrict__ bp, int nprob) {
-  extern __shared__ double smem[];
-  leaf_qr_body<WAVES, CPW, RPL>(A, lda, m, L, b, Rout, Tout, tauout, bp, nprob, blockIdx.x, smem);
-}
 
 // Packed column-major triangles in LDS: upper (r ≤ c) and strictly upper.
 __device__ __forceinline__ int pu(int r, int c) { return (c * (c + 1) >> 1) + r; }
@@ -478,40 +463,16 @@ __global__ void copy2d_kernel(const double* __restrict__ S, int64_t lds, double*
 // ===========================================================================
 // Launchers
 // ===========================================================================
-template <int WAVES, int CPW, int RPL>
-static int leaf_launch(cqr_ctx* c, double* A, int64_t lda, int64_t m, int L, int b,
-                       double* R, double* T, double* tau, const BatchProb* bp = nullptr, int nprob = 0) {
-  const size_t lds = sizeof(double) * ((size_t)b * b + 2 * 64 * RPL + 128);
-  auto k = leaf_qr_kernel<WAVES, CPW, RPL>;
-  CQR_TRY(set_max_lds(c, (const void*)k, 163840));
-  hipEvent_t ev = prof_begin(c);
-  hipLaunchKernelGGL(k, dim3(L), dim3(64 * WAVES), lds, c->stream, A, lda, m, L, b, R, T, tau, bp, nprob);
-  prof_end(c, ev, PK_LEAF, 2.0 * m * b * b - (2.0 / 3.0) * L * (double)b * b * b, 16.0 * m * b);
-  return check_launch(c, "leaf_qr");
-}
-
 // Batched: L = total leaves of the group, m = its total rows, rows = the
-// largest leaf of any problem (selects the register tile).
+// largest leaf of any problem.
 int leaf_qr_batched(cqr_ctx* c, double* Abase, int64_t total_m, int L, int64_t rows, int b, double* R, double* T,
                     double* tau, const BatchProb* bp, int nprob) {
-  if (b <= 16) return leaf_launch<4, 4, 16>(c, Abase, 0, total_m, L, b, R, T, tau, bp, nprob);
-  if (b <= 32) return rows <= 512 ? leaf_launch<8, 4, 8>(c, Abase, 0, total_m, L, b, R, T, tau, bp, nprob)
-                                  : leaf_launch<8, 4, 16>(c, Abase, 0, total_m, L, b, R, T, tau, bp, nprob);
-  if (b <= 64) return rows <= 256 ? leaf_launch<8, 8, 4>(c, Abase, 0, total_m, L, b, R, T, tau, bp, nprob)
-                                  : leaf_launch<8, 8, 8>(c, Abase, 0, total_m, L, b, R, T, tau, bp, nprob);
   return leaf16(c, Abase, 0, total_m, L, rows, b, R, T, tau, bp, nprob);
 }
 
 int leaf_qr(cqr_ctx* c, double* A, int64_t lda, int64_t m, int L, int b, double* R, double* T,
             double* tau) {
-  // rows per lane sized to the largest leaf (the register tile is RPL·64 rows)
-  const int64_t rows = (m + L - 1) / L;
-  if (b <= 16) return leaf_launch<4, 4, 16>(c, A, lda, m, L, b, R, T, tau);
-  if (b <= 32) return rows <= 512 ? leaf_launch<8, 4, 8>(c, A, lda, m, L, b, R, T, tau)
-                                  : leaf_launch<8, 4, 16>(c, A, lda, m, L, b, R, T, tau);
-  if (b <= 64) return rows <= 256 ? leaf_launch<8, 8, 4>(c, A, lda, m, L, b, R, T, tau)
-                                  : leaf_launch<8, 8, 8>(c, A, lda, m, L, b, R, T, tau);
-  return leaf16(c, A, lda, m, L, rows, b, R, T, tau, nullptr, 0);
+  return leaf16(c, A, lda, m, L, (m + L - 1) / L, b, R, T, tau, nullptr, 0);
 }
 
 int64_t leaf_capacity_rows(int64_t b) {
