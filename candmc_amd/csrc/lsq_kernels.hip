@@ -3,6 +3,7 @@
 // on A), element-wise updates and column norms.
 #include "cqr_device.h"
 #include "cqr_internal.h"
+#include "panel16.h"
 
 namespace cqr {
 
@@ -345,107 +346,133 @@ int launch_trsm_step(cqr_ctx* c, const double* R, int64_t ldr, int64_t n, const 
 // R(p, q)ᵀ·x_p) as each x_p is published, then forms x_q = op(R_qq⁻¹)·y_q
 // and publishes it (device-coherent stores, then flags[q] = 1).  Workgroup
 // ids follow the finishing order, so every block waits only on smaller ids
-// and dispatch order alone guarantees progress.  R's block for the next
-// dependency and R_qq⁻¹ are loaded into registers before each wait.  The
-// flags must be zero at launch; a wait that times out sets err[0] and the
-// block finishes (and publishes) with what it has.
-template <int NR>
+// and dispatch order alone guarantees progress.  The flags must be zero at
+// launch; a wait that times out sets err[0] and the block finishes (and
+// publishes) with what it has.
+//
+// Bound: the chain of blocks.  Products on FP64 MFMA tiles: wave w owns the
+// tile rows w and 7 − w of its block, whose tiles of R for the next dependency
+// and of R_qq⁻¹ are in registers before each wait, so that a link of the chain
+// is the hand-over and 100 MFMAs.  1100 columns (nine blocks), 5 right-hand
+// sides: 265 µs with a row of the block a thread (64 FMAs a right-hand side
+// and dependency, padded to 16), 56 µs here; 2048 columns, one: 174 → 130.
 __global__ void __launch_bounds__(256)
 trsm_chain_kernel(const double* __restrict__ R, int64_t ldr, int64_t n, const double* __restrict__ Rinv,
                   double* __restrict__ B, int64_t ldb, int nr, int trans, uint64_t* __restrict__ flags,
                   int* __restrict__ err) {
-  __shared__ double xs[128][NR + 1];
-  __shared__ double ys[128][NR + 1];
-  __shared__ double part[2][128][NR + 1];
+  __shared__ double xs[8 * P16_TILE], ys[8 * P16_TILE];
   __shared__ int s_err;
   const int nb = (int)((n + 127) / 128);
   const int q = trans ? (int)blockIdx.x : nb - 1 - (int)blockIdx.x;
-  const int t = threadIdx.x, r = t & 127, h = t >> 7, kb = h * 64;   // row of the block, half of the k range
+  const int tid = threadIdx.x, lane = tid & 63, w = wave_id();
+  const int c = lane & 15, g = lane >> 4;
   const int64_t jq = (int64_t)q * 128;
   const int bq = (int)min<int64_t>(128, n - jq);
-  for (int e = t; e < 128 * NR; e += 256) {
-    const int rr = e & 127, j = e >> 7;
-    ys[rr][j] = (rr < bq && j < nr) ? B[jq + rr + (int64_t)j * ldb] : 0.0;
-  }
-  if (t == 0) s_err = 0;
-  // op(R_qq⁻¹)(r, k) for this thread's half of k: upper (k ≥ r), or the
-  // transpose (k ≤ r)
-  const double* Ri = Rinv + (int64_t)q * 128 * 128;
-  double ri[64];
+  const dbl4 zero = {0.0, 0.0, 0.0, 0.0};
+  auto row_of = [&](int i) { return i ? 7 - w : w; };
+  // Tile (t, kt) as a left operand, element (r, k) at r·rs + k·cs; rows and
+  // columns past the ends come from the last one and are dropped or meet zeros.
+  auto fetch = [&](const double* p, int64_t rs, int64_t cs, int t, int kt, int rows, int cols) {
+    const double* a = p + min(16 * t + c, rows - 1) * rs;
+    dbl4 x;
 #pragma unroll
-  for (int u = 0; u < 64; ++u) {
-    const int k = kb + u;
-    const bool ok = r < bq && k < bq && (trans ? k <= r : k >= r);
-    ri[u] = Ri[ok ? (trans ? k + (int64_t)r * bq : r + (int64_t)k * bq) : 0];
-  }
-  const int ndep = trans ? q : nb - 1 - q;
-  double a[64];
-  auto load_block = [&](int i) {   // R's block against the i-th dependency
-    const int p = trans ? i : nb - 1 - i;
-    const int64_t jp = (int64_t)p * 128;
-    const int bp = (int)min<int64_t>(128, n - jp);
+    for (int v = 0; v < 4; ++v) x[v] = a[min(16 * kt + g + 4 * v, cols - 1) * cs];
+    return x;
+  };
+  if (tid == 0) s_err = 0;
+  // the strip's rows of a block: zero past its end and its right-hand sides
+  const double* Bc = B + (int64_t)min(c, nr - 1) * ldb;
+  dbl4 y[2];
 #pragma unroll
-    for (int u = 0; u < 64; ++u) {
-      const int k = kb + u;
-      const bool ok = r < bq && k < bp;
-      const int64_t idx = trans ? (jp + k) + (jq + r) * ldr : (jq + r) + (jp + k) * ldr;
-      a[u] = R[ok ? idx : 0];
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const int row = 16 * row_of(i) + g + 4 * v;
+      y[i][v] = row < bq && c < nr ? Bc[jq + row] : 0.0;
     }
+  // op(R_qq⁻¹): upper, or its transpose
+  const double* Ri = Rinv + (int64_t)q * 128 * 128;
+  dbl4 ri[2][8];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int kt = 0; kt < 8; ++kt)
+      if (trans ? kt <= row_of(i) : kt >= row_of(i))
+        ri[i][kt] = trans ? fetch(Ri, bq, 1, row_of(i), kt, bq, bq) : fetch(Ri, 1, bq, row_of(i), kt, bq, bq);
+  const int ndep = trans ? q : nb - 1 - q;
+  dbl4 a[2][8];
+  auto load_block = [&](int d) {   // R's block against the d-th dependency
+    const int64_t jp = (int64_t)(trans ? d : nb - 1 - d) * 128;
+    const int bp = (int)min<int64_t>(128, n - jp);
+    const double* p = trans ? R + jp + jq * ldr : R + jq + jp * ldr;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int kt = 0; kt < 8; ++kt)
+        a[i][kt] = trans ? fetch(p, ldr, 1, row_of(i), kt, bq, bp) : fetch(p, 1, ldr, row_of(i), kt, bq, bp);
   };
   if (ndep > 0) load_block(0);
-  for (int i = 0; i < ndep; ++i) {
-    const int p = trans ? i : nb - 1 - i;
+#pragma unroll 1
+  for (int d = 0; d < ndep; ++d) {
+    const int p = trans ? d : nb - 1 - d;
     const int64_t jp = (int64_t)p * 128;
     const int bp = (int)min<int64_t>(128, n - jp);
-    if (t == 0 && !s_err && !flag_wait(flags + p, 1, wait_limit(err))) s_err = 1;
-    __syncthreads();
-    for (int e = t; e < 128 * NR; e += 256) {
-      const int rr = e & 127, j = e >> 7;
-      xs[rr][j] = (rr < bp && j < nr) ? load_coherent(B + jp + rr + (int64_t)j * ldb) : 0.0;
-    }
-    __syncthreads();
-    double acc[NR];
+    if (tid == 0 && !s_err && !flag_wait(flags + p, 1, wait_limit(err))) s_err = 1;
+    __syncthreads();   // (xs has been read)
+    dbl4 x[2];
 #pragma unroll
-    for (int j = 0; j < NR; ++j) acc[j] = 0.0;
+    for (int i = 0; i < 2; ++i)
 #pragma unroll
-    for (int u = 0; u < 64; ++u) {
-      if (kb + u < bp) {
-#pragma unroll
-        for (int j = 0; j < NR; ++j) acc[j] += a[u] * xs[kb + u][j];
+      for (int v = 0; v < 4; ++v) {
+        const int row = 16 * row_of(i) + g + 4 * v;
+        x[i][v] = row < bp && c < nr ? load_coherent(Bc + jp + row) : 0.0;
       }
-    }
 #pragma unroll
-    for (int j = 0; j < NR; ++j) part[h][r][j] = acc[j];
+    for (int i = 0; i < 2; ++i) p16_store(xs + row_of(i) * P16_TILE, -x[i], lane);
     __syncthreads();
-    if (h == 0 && r < bq) {
 #pragma unroll
-      for (int j = 0; j < NR; ++j) ys[r][j] -= part[0][r][j] + part[1][r][j];
+    for (int kt = 0; kt < 8; ++kt) {
+      const dbl4 xk = p16_load(xs + kt * P16_TILE, lane);
+#pragma unroll
+      for (int v = 0; v < 4; ++v)
+#pragma unroll
+        for (int i = 0; i < 2; ++i) y[i] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[i][kt][v], xk[v], y[i], 0, 0, 0);
     }
-    if (i + 1 < ndep) load_block(i + 1);   // in flight during the next wait
-  }
-  __syncthreads();
-  double acc[NR];
-#pragma unroll
-  for (int j = 0; j < NR; ++j) acc[j] = 0.0;
-#pragma unroll
-  for (int u = 0; u < 64; ++u) {
-    const int k = kb + u;
-    if (k < bq && r < bq && (trans ? k <= r : k >= r)) {
-#pragma unroll
-      for (int j = 0; j < NR; ++j) acc[j] += ri[u] * ys[k][j];
-    }
+    if (d + 1 < ndep) load_block(d + 1);   // in flight during the next wait
   }
 #pragma unroll
-  for (int j = 0; j < NR; ++j) part[h][r][j] = acc[j];
-  __syncthreads();
-  if (h == 0 && r < bq) {
+  for (int i = 0; i < 2; ++i) {
 #pragma unroll
-    for (int j = 0; j < NR; ++j)
-      if (j < nr) store_coherent(B + jq + r + (int64_t)j * ldb, part[0][r][j] + part[1][r][j]);
+    for (int v = 0; v < 4; ++v) y[i][v] = 16 * row_of(i) + g + 4 * v < bq ? y[i][v] : 0.0;
+    p16_store(ys + row_of(i) * P16_TILE, y[i], lane);
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int t = row_of(i);
+    dbl4 x0 = zero, x1 = zero;
+#pragma unroll
+    for (int kt = 0; kt < 8; ++kt)
+      if (trans ? kt <= t : kt >= t) {
+        if (kt == t)
+#pragma unroll
+          for (int v = 0; v < 4; ++v) ri[i][kt][v] = (trans ? g + 4 * v <= c : g + 4 * v >= c) ? ri[i][kt][v] : 0.0;
+        const dbl4 yk = p16_load(ys + kt * P16_TILE, lane);
+#pragma unroll
+        for (int v = 0; v < 4; v += 2) {
+          x0 = __builtin_amdgcn_mfma_f64_16x16x4f64(ri[i][kt][v], yk[v], x0, 0, 0, 0);
+          x1 = __builtin_amdgcn_mfma_f64_16x16x4f64(ri[i][kt][v + 1], yk[v + 1], x1, 0, 0, 0);
+        }
+      }
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const int row = 16 * t + g + 4 * v;
+      if (row < bq && c < nr) store_coherent(B + jq + row + (int64_t)c * ldb, x0[v] + x1[v]);
+    }
   }
   wait_memory();   // this wave's x_q stores have reached memory
   __syncthreads();
-  if (t == 0) {
+  if (tid == 0) {
     if (s_err) err[0] = 1;
     flag_store(flags + q, 1);
   }
@@ -457,16 +484,12 @@ int launch_trsm_chain(cqr_ctx* c, const double* R, int64_t ldr, int64_t n, const
   if (nr < 1 || nr > 16 || nb < 1 || nb > CQR_TRSM_MAX_BLOCKS)
     return set_err(c, CQR_ERR_UNSUPPORTED, "trsm chain: %d columns, %lld blocks", nr, (long long)nb);
   CQR_TRY(launch_fill2d(c, reinterpret_cast<double*>(c->d_sflags), nb, nb, 1, 0.0));   // all-zero bits
-  auto run = [&](auto k) -> int {
-    SpinScope gate(c, (const void*)k, nb, 256, 0);
+  {
+    SpinScope gate(c, (const void*)trsm_chain_kernel, nb, 256, 0);
     CQR_TRY(gate.status());
-    hipLaunchKernelGGL(k, dim3((unsigned)nb), dim3(256), 0, c->stream, R, ldr, n, Rinv, B, ldb, nr, trans,
+    hipLaunchKernelGGL(trsm_chain_kernel, dim3((unsigned)nb), dim3(256), 0, c->stream, R, ldr, n, Rinv, B, ldb, nr, trans,
                        c->d_sflags, c->d_terr);
-    return CQR_OK;
-  };
-  if (nr == 1) CQR_TRY(run(trsm_chain_kernel<1>));
-  else if (nr <= 4) CQR_TRY(run(trsm_chain_kernel<4>));
-  else CQR_TRY(run(trsm_chain_kernel<16>));
+  }
   return check_launch(c, "trsm_chain");
 }
 
