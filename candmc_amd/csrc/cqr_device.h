@@ -234,33 +234,6 @@ __device__ inline dbl4 mfma_tile16(const FX& x, const FY& y, int k0, int k1, int
   return acc;
 }
 
-// Same tile with the k steps dealt round-robin to four accumulators, so
-// consecutive MFMAs are independent and issue back to back instead of each
-// waiting for the previous result (the chains are summed at the end).  The
-// accessors are called for every k of a 64-wide chunk, also k ≥ k1: they
-// must stay in bounds there and return 0 (branch-free accessors let the
-// 32 loads of a chunk issue together).
-template <class FX, class FY>
-__device__ inline dbl4 mfma_tile16_acc4(const FX& x, const FY& y, int k0, int k1, int lane) {
-  const int r = lane & 15, q = lane >> 4;
-  dbl4 acc[4];
-#pragma unroll
-  for (int a = 0; a < 4; ++a) acc[a] = dbl4{0.0, 0.0, 0.0, 0.0};
-  for (int kc = k0; kc < k1; kc += 64) {
-    double xa[16], yb[16];
-#pragma unroll
-    for (int s = 0; s < 16; ++s) {
-      const int k = kc + 4 * s;
-      xa[s] = x(r, k + q);
-      yb[s] = y(k + q, r);
-    }
-#pragma unroll
-    for (int s = 0; s < 16; ++s)
-      if (kc + 4 * s < k1) acc[s & 3] = __builtin_amdgcn_mfma_f64_16x16x4f64(yb[s], xa[s], acc[s & 3], 0, 0, 0);
-  }
-  return (acc[0] + acc[1]) + (acc[2] + acc[3]);
-}
-
 // ---------------------------------------------------------------------------
 // In-LDS inverse of an upper triangular b×b matrix (column-major, ld),
 // whole workgroup.  On entry the strictly upper part of M holds N and

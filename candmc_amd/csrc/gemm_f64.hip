@@ -11,6 +11,7 @@
 // attribute time to each use.
 #include "cqr_device.h"
 #include "cqr_internal.h"
+#include "panel16.h"
 
 #include <type_traits>
 
@@ -372,10 +373,11 @@ static int choose_splits(int64_t m, int64_t n, int64_t k, int64_t* kchunk) {
 
 // Small products (m, n, k ≤ 256: the b×b triangles of T, W, L⁻ᵀ and the
 // b-wide Z' = Tᵀ·Z): one wave per 16×16 output tile, operands read straight
-// from memory (they sit in L2) with the structural masks applied per
-// element on the stored coordinates, FP64 MFMA with four accumulator
-// chains.  A 128×128×128 product is 64 single-wave workgroups instead of
-// one 256-thread tile walking eight LDS slabs.
+// from memory (they sit in L2), 128 values of k of both in flight at once,
+// with the structural masks applied per element on the stored coordinates.
+// A 128×128×128 product is 64 single-wave workgroups instead of one
+// 256-thread tile walking eight LDS slabs.  Bound: load latency; 32×64×160
+// takes 15 µs (18 with 64 values of k in flight).
 struct SmallArgs {
   int m, n, k, ta, tb, smA, smB;
   double alpha, beta;
@@ -390,21 +392,28 @@ struct SmallArgs {
 __global__ void __launch_bounds__(64) small_gemm_kernel(SmallArgs g) {
   const int lane = threadIdx.x;
   const int i0 = blockIdx.x * 16, j0 = blockIdx.y * 16;
-  auto x = [&](int r, int kk) {   // op(A)(i0 + r, kk)
-    const int i = i0 + r;
-    const bool ok = i < g.m && kk < g.k;
-    const int64_t sr = g.ta ? kk : i, sc = g.ta ? i : kk;
-    const double v = g.A[ok ? sr + sc * g.lda : 0];
-    return ok ? gmask(v, sr, sc, g.smA) : 0.0;
-  };
-  auto y = [&](int kk, int cc) {  // op(B)(kk, j0 + cc)
-    const int j = j0 + cc;
-    const bool ok = j < g.n && kk < g.k;
-    const int64_t sr = g.tb ? j : kk, sc = g.tb ? kk : j;
-    const double v = g.B[ok ? sr + sc * g.ldb : 0];
-    return ok ? gmask(v, sr, sc, g.smB) : 0.0;
-  };
-  const dbl4 acc = mfma_tile16_acc4(x, y, 0, g.k, lane);
+  // the operands of 128 values of k are in flight before the first is used
+  const int c = lane & 15, q = lane >> 4, ia = i0 + c, jb = j0 + c;
+  dbl4 acc0 = {0.0, 0.0, 0.0, 0.0}, acc1 = acc0;
+  for (int k0 = 0; k0 < g.k; k0 += 128) {
+    double x[32], y[32];
+#pragma unroll
+    for (int s = 0; s < 32; ++s) {
+      const int kk = k0 + 4 * s + q;
+      x[s] = g.A[ia < g.m && kk < g.k ? (g.ta ? kk + ia * g.lda : ia + kk * g.lda) : 0];
+      y[s] = g.B[jb < g.n && kk < g.k ? (g.tb ? jb + kk * g.ldb : kk + jb * g.ldb) : 0];
+    }
+#pragma unroll
+    for (int s = 0; s < 32; ++s) {
+      if (k0 + 4 * s >= g.k) continue;
+      const int kk = k0 + 4 * s + q;
+      const double a = ia < g.m && kk < g.k ? gmask(x[s], g.ta ? kk : ia, g.ta ? ia : kk, g.smA) : 0.0;
+      const double b = jb < g.n && kk < g.k ? gmask(y[s], g.tb ? jb : kk, g.tb ? kk : jb, g.smB) : 0.0;
+      if (s & 1) acc1 = __builtin_amdgcn_mfma_f64_16x16x4f64(b, a, acc1, 0, 0, 0);
+      else acc0 = __builtin_amdgcn_mfma_f64_16x16x4f64(b, a, acc0, 0, 0, 0);
+    }
+  }
+  const dbl4 acc = acc0 + acc1;
   const int i = i0 + (lane & 15);
 #pragma unroll
   for (int v = 0; v < 4; ++v) {
@@ -431,60 +440,64 @@ static int launch_small(cqr_ctx* c, int ta, int tb, int64_t m, int64_t n, int64_
 
 // Products with few columns (n ≤ 16; m, k ≤ 256: the solves' R blocks and
 // the b×b×nrhs steps of the Q application): one workgroup, op(B) staged in
-// LDS, one thread per output row with NR accumulators, reading its row of
-// op(A) straight from memory 64 values at a time (all 64 loads in flight
-// before the first is used).  Every element of B is read before any element
-// of C is written, so C may alias B.
-template <int NR>
+// LDS as a strip of 16 columns, FP64 MFMA tiles of op(A) straight from memory,
+// a wave's row of up to eight tiles in flight at once.  Every element of B is
+// read before any element of C is written, so C may alias B.  Bound: the
+// latency of two dependent loads; 128×128×5 takes 14 µs (34 with a row a
+// thread and FMAs for 16 columns).
 __global__ void __launch_bounds__(256) small_thin_kernel(SmallArgs g) {
-  constexpr int KC = 64;
-  __shared__ double Bs[256][NR + 1];
-  const int t = threadIdx.x;
-  {  // Bs[kk][j] = op(B)(kk, j): thread t loads row kk = t
-    double v[NR];
+  __shared__ double Bs[256 * P16_LD];
+  const int t = threadIdx.x, lane = t & 63, w = wave_id(), c = lane & 15, q = lane >> 4;
+  {  // thread t loads row kk = t of op(B)
+    double v[16];
 #pragma unroll
-    for (int j = 0; j < NR; ++j) {
+    for (int j = 0; j < 16; ++j) {
       const bool ok = t < g.k && j < g.n;
       const int64_t sr = g.tb ? j : t, sc = g.tb ? t : j;
       v[j] = g.B[ok ? sr + sc * g.ldb : 0];
     }
 #pragma unroll
-    for (int j = 0; j < NR; ++j) {
+    for (int j = 0; j < 16; ++j) {
       const bool ok = t < g.k && j < g.n;
       const int64_t sr = g.tb ? j : t, sc = g.tb ? t : j;
-      if (t < g.k) Bs[t][j] = ok ? gmask(v[j], sr, sc, g.smB) : 0.0;
+      Bs[t * P16_LD + j] = ok ? gmask(v[j], sr, sc, g.smB) : 0.0;
     }
   }
   __syncthreads();
-  if (t >= g.m) return;
-  double acc[NR];
+  for (int i0 = 16 * w; i0 < g.m; i0 += 64) {
+    dbl4 acc0 = {0.0, 0.0, 0.0, 0.0}, acc1 = acc0;
+    const int i = i0 + c;
+    for (int k0 = 0; k0 < g.k; k0 += 128) {
+      dbl4 x[8];
 #pragma unroll
-  for (int j = 0; j < NR; ++j) acc[j] = 0.0;
-  for (int k0 = 0; k0 < g.k; k0 += KC) {
-    double v[KC];
+      for (int kt = 0; kt < 8; ++kt)
 #pragma unroll
-    for (int q = 0; q < KC; ++q) {
-      const int kk = k0 + q;
-      const bool ok = kk < g.k;
-      const int64_t sr = g.ta ? kk : t, sc = g.ta ? t : kk;
-      v[q] = g.A[ok ? sr + sc * g.lda : 0];
+        for (int v = 0; v < 4; ++v) {
+          const int kk = k0 + 16 * kt + q + 4 * v;
+          const int64_t sr = g.ta ? kk : i, sc = g.ta ? i : kk;
+          x[kt][v] = g.A[i < g.m && kk < g.k ? sr + sc * g.lda : 0];
+        }
+#pragma unroll
+      for (int kt = 0; kt < 8; ++kt)
+        if (k0 + 16 * kt < g.k) {
+          const dbl4 y = p16_load(Bs + (k0 + 16 * kt) * P16_LD, lane);
+#pragma unroll
+          for (int v = 0; v < 4; ++v) {
+            const int kk = k0 + 16 * kt + q + 4 * v;
+            const int64_t sr = g.ta ? kk : i, sc = g.ta ? i : kk;
+            const double a = i < g.m && kk < g.k ? gmask(x[kt][v], sr, sc, g.smA) : 0.0;
+            if (v & 1) acc1 = __builtin_amdgcn_mfma_f64_16x16x4f64(a, y[v], acc1, 0, 0, 0);
+            else acc0 = __builtin_amdgcn_mfma_f64_16x16x4f64(a, y[v], acc0, 0, 0, 0);
+          }
+        }
     }
 #pragma unroll
-    for (int q = 0; q < KC; ++q) {
-      const int kk = k0 + q;
-      if (kk < g.k) {
-        const int64_t sr = g.ta ? kk : t, sc = g.ta ? t : kk;
-        const double a = gmask(v[q], sr, sc, g.smA);
-#pragma unroll
-        for (int j = 0; j < NR; ++j) acc[j] += a * Bs[kk][j];
-      }
+    for (int v = 0; v < 4; ++v) {
+      const int row = i0 + q + 4 * v;
+      if (row >= g.m || c >= g.n) continue;
+      double* cp = g.C + row + (int64_t)c * g.ldc;
+      *cp = g.alpha * (acc0[v] + acc1[v]) + (g.beta != 0.0 ? g.beta * *cp : 0.0);
     }
-  }
-#pragma unroll
-  for (int j = 0; j < NR; ++j) {
-    if (j >= g.n) continue;
-    double* cp = g.C + t + (int64_t)j * g.ldc;
-    *cp = g.alpha * acc[j] + (g.beta != 0.0 ? g.beta * *cp : 0.0);
   }
 }
 
@@ -499,9 +512,7 @@ int launch_small_thin(cqr_ctx* c, int ta, int tb, int64_t m, int64_t n, int64_t 
   g.m = (int)m; g.n = (int)n; g.k = (int)k; g.ta = ta; g.tb = tb; g.smA = smA; g.smB = smB;
   g.alpha = alpha; g.beta = beta; g.A = A; g.lda = lda; g.B = B; g.ldb = ldb; g.C = C; g.ldc = ldc;
   hipEvent_t ev = prof_begin(c);
-  if (n == 1) hipLaunchKernelGGL(small_thin_kernel<1>, dim3(1), dim3(256), 0, c->stream, g);
-  else if (n <= 4) hipLaunchKernelGGL(small_thin_kernel<4>, dim3(1), dim3(256), 0, c->stream, g);
-  else hipLaunchKernelGGL(small_thin_kernel<16>, dim3(1), dim3(256), 0, c->stream, g);
+  hipLaunchKernelGGL(small_thin_kernel, dim3(1), dim3(256), 0, c->stream, g);
   prof_end(c, ev, kind, 2.0 * m * n * k, 8.0 * ((double)m * k + (double)k * n + 2.0 * m * n));
   return check_launch(c, "small_thin");
 }
