@@ -201,10 +201,18 @@ __device__ __forceinline__ void p16_larfg(double alpha, double ss, double& beta,
 // place in Vs).  Each part publishes its share of a column's dot products in
 // `ex` (two buffers of PARTS + 1 rows of sixteen, the last one the pivot row),
 // and after a workgroup barrier all of them form the same reflector.
-template <int RT, bool NODE, int PARTS = 1>
+//
+// With GLOB (a leaf of one strip) nobody else reads the vectors: the tiles stay
+// in registers, scaled in place, and the slow path (`taken`) works on the leaf
+// in memory, which still holds the strip, and leaves the vectors there; col is
+// this lane's column, of `rows` rows (none past the matrix's last column).
+template <int RT, bool NODE, int PARTS = 1, bool GLOB = false>
 struct Panel16 {
   double* ex;
   int part = 0;
+  double* col;
+  int rows;
+  bool taken = false;
   // the tiles [H, RT) are skipped as a whole once they are zero (never in a
   // tall leaf, whose parts stay full)
   static constexpr int H = PARTS > 1 ? RT : RT > 8 ? 8 : RT > 4 ? 4 : RT;
@@ -302,12 +310,26 @@ struct Panel16 {
   }
 
   // The whole panel with dlarfg's general semantics (rescaling, zero and
-  // non-finite columns), in LDS: nt tiles in Vs, the pivot tile in Ds.
-  __device__ __forceinline__ static void slow(double* Vs, double* Ds, double* Zs, int nt, int nb, double& tau_out) {
+  // non-finite columns), in memory: nt tiles in Vs, the pivot tile in Ds.
+  __device__ __forceinline__ void slow(double* Vs, double* Ds, double* Zs, int nt, int nb, double& tau_out) const {
     const int lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
     auto sync = []() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup"); };
     // element v of this lane's column in tile t (t < 0: the pivot tile)
-    auto at = [&](int t, int v) -> double& { return (t < 0 ? Ds : Vs + t * P16_TILE)[(g + 4 * v) * P16_LD + c]; };
+    auto place = [&](int t, int v) -> double* {
+      if (GLOB && t >= 0) {
+        const int row = 16 * (t + 1) + 4 * g + v;
+        return row < rows ? col + row : nullptr;
+      }
+      return (t < 0 ? Ds : Vs + t * P16_TILE) + (g + 4 * v) * P16_LD + c;
+    };
+    auto at = [&](int t, int v) {
+      const double* q = place(t, v);
+      return !GLOB || q ? *q : 0.0;
+    };
+    auto put = [&](int t, int v, double x) {
+      double* q = place(t, v);
+      if (!GLOB || q) *q = x;
+    };
     auto pivot_row = [&](int v) { return NODE ? g + 4 * v : 4 * g + v; };
     const int t0 = NODE ? 0 : -1;
     double tau = 0.0;
@@ -342,7 +364,7 @@ struct Panel16 {
             if (below(t, v)) {
               double x = at(t, v);
               for (int k = 0; k < h.knt; ++k) x *= 0x1p969;
-              at(t, v) = x * h.scal;
+              put(t, v, x * h.scal);
             }
       sync();
       double s = 0.0;
@@ -357,7 +379,7 @@ struct Panel16 {
       for (int t = t0; t < nt; ++t)
         for (int v = 0; v < 4; ++v) {
           const double x = __shfl(at(t, v), src);
-          if (c > j && below(t, v)) at(t, v) -= f * x;
+          if (c > j && below(t, v)) put(t, v, at(t, v) - f * x);
         }
       if (g == 0) {
         Ds[jr * P16_LD + c] = c > j ? p - f : (c == j ? h.beta : p);
@@ -408,9 +430,10 @@ struct Panel16 {
     // kept for the slow path: straight-line columns with one test at the end
     // cost less than a way out of every column
     p16_store(Ds, D, lane);
+    if constexpr (!GLOB)
 #pragma unroll
-    for (int t = 0; t < RT; ++t)
-      if (t < H || nact > H) p16_store(Vs + t * P16_TILE, a[t], lane);
+      for (int t = 0; t < RT; ++t)
+        if (t < H || nact > H) p16_store(Vs + t * P16_TILE, a[t], lane);
     double* Zc = Zs + c;
 #pragma unroll
     for (int q = 0; q < P16; ++q) pr[q] = Ds[trow_of(q) * P16_LD + c];
@@ -425,15 +448,20 @@ struct Panel16 {
     P16_STEP(0) P16_STEP(1) P16_STEP(2) P16_STEP(3) P16_STEP(4) P16_STEP(5) P16_STEP(6) P16_STEP(7)
     P16_STEP(8) P16_STEP(9) P16_STEP(10) P16_STEP(11) P16_STEP(12) P16_STEP(13) P16_STEP(14) P16_STEP(15)
 #undef P16_STEP
+    if constexpr (GLOB)   // (without meaning on the slow path)
+#pragma unroll
+      for (int t = 0; t < RT; ++t) a[t] *= scale;
     // the fast range: ‖x‖² in (2^-200, 2^200), |alpha| < 2^200, dots far from
     // overflow; a NaN or infinity fails it
     if (__builtin_amdgcn_ballot_w64(!(ssv > 0x1p-200 && ssv < 0x1p200 && fabs(alv) < 0x1p200 && smax < 0x1p800)) != 0) {
+      taken = true;
       if (PARTS > 1 && part != 0) return;
       slow(Vs, Ds, Zs, PARTS > 1 ? RT + 16 * (PARTS - 1) : nact > H ? RT : H, nb, tau);
     } else {
+      if constexpr (!GLOB)
 #pragma unroll
-      for (int t = 0; t < RT; ++t)
-        if (t < H || nact > H) p16_store(Vs + t * P16_TILE, a[t] * scale, lane);
+        for (int t = 0; t < RT; ++t)
+          if (t < H || nact > H) p16_store(Vs + t * P16_TILE, a[t] * scale, lane);
       if (PARTS > 1 && part != 0) {
         p16_store(Ds, dbl4{pr[0], pr[1], pr[2], pr[3]} * scale, lane);
         return;

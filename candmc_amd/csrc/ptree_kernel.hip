@@ -247,16 +247,19 @@ __device__ __forceinline__ void leaf16_body(double* __restrict__ A, int64_t lda,
 // ---------------------------------------------------------------------------
 // A leaf taller than a wave's registers (r ≤ 256·P rows, b ≤ 16·S columns):
 // P waves share a strip, 256 rows each, the first of them with the pivot
-// tile.  They factor a panel together (a barrier a column) and add their shares of each product in LDS (X), so the steps run
-// one after another, with one panel of V in LDS.  Three loops rather than one
-// with roles: the factor() of the strip's own panel then stands in no loop,
-// where its registers spilled.  512×64 leaves take 0.11 ms (0.125 with a
-// reflector at a time over 64-row lanes); hh_recon_qr of 65536×16 234 →
-// 162 µs, ×32 328 → 245, 16384×64 458 → 321 (with the other kernels' gains).
+// tile.  They factor a panel together (a barrier a column) and add their
+// shares of each product in LDS (X), so the steps run one after another, with
+// one panel of V in LDS.  Three loops rather than one with roles: the factor()
+// of the strip's own panel then stands in no loop, where its registers
+// spilled.  512×64 leaves take 0.11 ms (0.125 with a reflector at a time over
+// 64-row lanes); hh_recon_qr of 65536×16 234 → 153 µs, ×32 328 → 245,
+// 16384×64 458 → 321 (with the other kernels' gains).  A single strip (b ≤ 16)
+// keeps its vectors in registers, so that two or four leaves share a CU: 4500
+// leaves of 1024×16 take 0.46 ms, 0.70 with V in 143 KB of LDS, a leaf a CU.
 // ---------------------------------------------------------------------------
 template <int S, int P>
 constexpr int tall_smem_doubles() {
-  return (16 * P + S * (S + 1) / 2 + 1 + (S - 1) * P) * P16_TILE + 2 * P16 * (P + 1);
+  return ((S > 1 ? 16 * P : P - 1) + S * (S + 1) / 2 + 1 + (S - 1) * P) * P16_TILE + 2 * P16 * (P + 1);
 }
 
 template <int S, int P>
@@ -280,8 +283,9 @@ __device__ __forceinline__ void leaf16_tall_body(double* __restrict__ A, int64_t
   double* Rl = Rout + (int64_t)gleaf * bb;
   double* Tl = Tout + (int64_t)gleaf * bb;
   double* taul = tauout + (int64_t)gleaf * b;
-  double* Vk = smem;                              // the panel, tile by tile
-  double* Ts = Vk + 16 * P * P16_TILE;            // tiles of T, and one for the pivot tile
+  // the panel, tile by tile; of a single strip only a tile for each low part's D
+  double* Vk = smem;
+  double* Ts = Vk + (S > 1 ? 16 * P : P - 1) * P16_TILE;   // tiles of T, and one for the pivot tile
   double* X = Ts + (S * (S + 1) / 2 + 1) * P16_TILE;
   double* ex = X + (S - 1) * P * P16_TILE;
 
@@ -313,7 +317,7 @@ __device__ __forceinline__ void leaf16_tall_body(double* __restrict__ A, int64_t
     zero_below(Rl, b, strip, lane);
     zero_below(Tl, b, strip, lane);
   }
-  double* Vp = Vk + 16 * part * P16_TILE;         // this part's tiles of the panel
+  double* Vp = Vk + (S > 1 ? 16 * part : part - 1) * P16_TILE;   // this part's tiles of the panel
   auto panel = [&](int k) {                       // another strip's panel: its columns, then V and T_kk are there
     for (int j = 16 * k; j < min(b, 16 * k + 16); ++j) __syncthreads();
     __syncthreads();
@@ -363,20 +367,24 @@ __device__ __forceinline__ void leaf16_tall_body(double* __restrict__ A, int64_t
     __syncthreads();
   }
   if (strip >= nblk) return;                      // (no barrier is left)
+  bool taken = false;                             // the vectors are in memory already
   {
     const int k = strip;
     __builtin_amdgcn_s_setprio(3);
-    Panel16<NB, false, P> F;
+    Panel16<NB, false, P, S == 1> F;
+    F.col = Ac - 4 * g;
+    F.rows = colok ? r : 0;
     F.ex = ex;
     F.part = part;
     F.factor(D, a, NB, min(P16, b - 16 * k), lane, Ts + p16_slot(k, k), Vp + P16_TILE,
              part == 0 ? Ts + p16_slot(0, S) : Vp);
     if (part == 0) {
+      if (S > 1)
 #pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const int row = 4 * g + v;
-        Vk[(g + 4 * v) * P16_LD + c] = row > c ? D[v] : (row == c ? 1.0 : 0.0);
-      }
+        for (int v = 0; v < 4; ++v) {
+          const int row = 4 * g + v;
+          Vk[(g + 4 * v) * P16_LD + c] = row > c ? D[v] : (row == c ? 1.0 : 0.0);
+        }
       if (g == 0 && colok) taul[col] = F.tau;
     }
     __builtin_amdgcn_s_setprio(0);
@@ -384,9 +392,14 @@ __device__ __forceinline__ void leaf16_tall_body(double* __restrict__ A, int64_t
     __syncthreads();
     // the scaled vectors back from LDS
     if (part == 0) put_t_tile(Tl, b, k, k, p16_load(Ts + p16_slot(k, k), lane), lane);
-    else D = p16_load(Vp, lane);
+    if constexpr (S > 1) {
+      if (part != 0) D = p16_load(Vp, lane);
 #pragma unroll
-    for (int t = 0; t < NB; ++t) a[t] = p16_load(Vp + (t + 1) * P16_TILE, lane);
+      for (int t = 0; t < NB; ++t) a[t] = p16_load(Vp + (t + 1) * P16_TILE, lane);
+    } else {
+      if (part != 0) D = p16_load(Vp, lane);
+      taken = F.taken;
+    }
     finish(k);
     __syncthreads();
   }
@@ -412,7 +425,7 @@ __device__ __forceinline__ void leaf16_tall_body(double* __restrict__ A, int64_t
     put_t_tile(Tl, b, strip, nblk - 1, p16_tcol(Ts, strip, nblk - 1, lane), lane);
   }
   // the rows below the last panel's block
-  if (strip < nblk) {
+  if (!taken) {
     const int t0 = part == 0 ? nblk : 0;
     p16_rows_store(Ac + 16 * t0, D, rg - 16 * t0, colok);
 #pragma unroll
@@ -587,7 +600,7 @@ leaf16_kernel(double* __restrict__ A, int64_t lda, int64_t m, int L, int b, doub
 }
 
 template <int S, int P>
-__global__ void __launch_bounds__(64 * S * P)
+__global__ void __launch_bounds__(64 * S * P) __attribute__((amdgpu_waves_per_eu(2)))
 leaf16_tall_kernel(double* __restrict__ A, int64_t lda, int64_t m, int L, int b, double* __restrict__ Rout,
                    double* __restrict__ Tout, double* __restrict__ tauout, const BatchProb* __restrict__ bp, int nprob) {
   extern __shared__ double smem[];
