@@ -633,8 +633,7 @@ int wy_update_ws(cqr_ctx* c, const double* Y, int64_t ldy, int y_implicit, const
 // Trailing update with an explicit unit-lower Y (Ye, m×b, ld m) and
 // YT = Ye·Tᵀ-factor product (m×b, ld m, i.e. Ye·Tt): A (m×n) −= YT·(Yeᵀ·A).
 // No structural masks remain, so both products are plain: Z = Yeᵀ·A on the
-// lean kernel (split-K, from three column tiles on) or the general one, and
-// the update through the vendor BLAS.
+// lean kernel (split-K) or the general one, and the update on upd_gemm_f64.
 // Z (b×n, in ws) = Yᵀ·A: the first product of the explicit update.
 int wy_explicit_yta(cqr_ctx* c, const double* Ye, int64_t m, int64_t n, int b, const double* A, int64_t lda,
                     double* ws, int prec, double** Zout) {

@@ -1,5 +1,5 @@
 // Panel kernels of the CA-QR hot path for gfx950 (FP64):
-//   tree_node     K2  QR of stacked triangles [R_top; R_bot] (dtpqrt l=b)
+//   tree_node     QR of stacked triangles [R_top; R_bot] (dtpqrt l=b)
 //   bgemm         small batched GEMMs for the reverse tree, the per-leaf
 //                 block-reflector products and the Y formation
 // plus element-wise helpers.  Leaves are contiguous row blocks
@@ -10,7 +10,6 @@
 #include "cqr_internal.h"
 
 namespace cqr {
-
 
 // Loop over the entries (rr, cc) of a b×b matrix: waves over columns, lanes
 // over rows (no integer division; coalesced along columns).
@@ -23,7 +22,7 @@ __device__ __forceinline__ int pu(int r, int c) { return (c * (c + 1) >> 1) + r;
 __device__ __forceinline__ int psu(int r, int c) { return (c * (c - 1) >> 1) + r; }
 
 // ---------------------------------------------------------------------------
-// K2: one tree level.  Node z stacks R of receiver z on R of sender
+// One tree level.  Node z stacks R of receiver z on R of sender
 // z + ceil(n/2) and computes its QR like dtpqrt with l = b: the reflector
 // for column i is [e_i; x] with x = R_bot(0:i, i), so R_bot becomes V2
 // (upper triangular, in registers as in K1) and R_top (packed in LDS)
