@@ -164,9 +164,11 @@ __device__ __forceinline__ void p16_fma_bc(double& acc, double z, double t) {
 // sqrt and the two reciprocals of dlarfg for ss = ‖x‖² in (2^-200, 2^200)
 // and |alpha| < 2^200: beta = −sign(alpha)·sqrt(alpha² + ss) by the
 // Goldschmidt iteration from the hardware's reciprocal square root with two
-// residual corrections; no operand scaling is needed in this range.
+// residual corrections; no operand scaling is needed in this range.  ss = 0
+// stands for a zero x: H = I, beta = alpha and tau = 0, with scal and rb finite
+// (they meet zeros only).
 __device__ __forceinline__ void p16_larfg(double alpha, double ss, double& beta, double& tau, double& scal, double& rb) {
-  const double x = fma(alpha, alpha, ss);
+  const double x = fmax(fma(alpha, alpha, ss), 0x1p-400);
   const double y = __builtin_amdgcn_rsq(x);
   double g = x * y, h = 0.5 * y;
   const double r = fma(-h, g, 0.5);
@@ -174,12 +176,13 @@ __device__ __forceinline__ void p16_larfg(double alpha, double ss, double& beta,
   g = fma(g, r, g);
   g = fma(fma(-g, g, x), h, g);
   g = fma(fma(-g, g, x), h, g);
-  beta = -copysign(g, alpha);
-  // 1/beta from the refined reciprocal root h ≈ 1/(2g)
+  const double bt = -copysign(g, alpha);
+  // 1/bt from the refined reciprocal root h ≈ 1/(2g)
   double q = h + h;
   q = fma(q, fma(-g, q, 1.0), q);
-  rb = copysign(q, beta);
-  scal = recip_nr(alpha - beta);
+  rb = copysign(q, bt);
+  scal = recip_nr(alpha - bt);
+  beta = ss == 0.0 ? alpha : bt;
   tau = (beta - alpha) * rb;
 }
 
@@ -448,12 +451,36 @@ struct Panel16 {
     P16_STEP(0) P16_STEP(1) P16_STEP(2) P16_STEP(3) P16_STEP(4) P16_STEP(5) P16_STEP(6) P16_STEP(7)
     P16_STEP(8) P16_STEP(9) P16_STEP(10) P16_STEP(11) P16_STEP(12) P16_STEP(13) P16_STEP(14) P16_STEP(15)
 #undef P16_STEP
+    // the fast range: ‖x‖² in (2^-200, 2^200) or x = 0, |alpha| < 2^200, dots
+    // far from overflow; a NaN or infinity fails it
+    bool bad = !((ssv > 0x1p-200 && ssv < 0x1p200) || ssv == 0.0) || !(fabs(alv) < 0x1p200 && smax < 0x1p800);
+    if (__builtin_amdgcn_ballot_w64(ssv == 0.0) != 0) {
+      // really nothing there, or entries too small to square?  (they are as
+      // their column's own step found them)
+      double nz = 0.0;
+#pragma unroll
+      for (int t = 0; t < RT; ++t)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) nz = fmax(nz, fabs(a[t][v]));
+      if (!NODE)
+#pragma unroll
+        for (int q = 0; q < P16; ++q) nz = fmax(nz, (PARTS > 1 && part != 0 ? q < 4 : q > c) ? fabs(pr[q]) : 0.0);
+      bad |= ssv == 0.0 && nz > 0.0;
+    }
+    bool redo = __builtin_amdgcn_ballot_w64(bad) != 0;
+    if constexpr (PARTS > 1) {                    // one decision for all parts
+      double* E = ex + (nb & 1) * (P16 * (PARTS + 1));
+      if (lane == 0) E[part] = redo ? 1.0 : 0.0;
+      __syncthreads();
+      redo = false;
+#pragma unroll
+      for (int q = 0; q < PARTS; ++q) redo |= E[q] != 0.0;
+      redo = __builtin_amdgcn_readfirstlane(redo) != 0;
+    }
     if constexpr (GLOB)   // (without meaning on the slow path)
 #pragma unroll
       for (int t = 0; t < RT; ++t) a[t] *= scale;
-    // the fast range: ‖x‖² in (2^-200, 2^200), |alpha| < 2^200, dots far from
-    // overflow; a NaN or infinity fails it
-    if (__builtin_amdgcn_ballot_w64(!(ssv > 0x1p-200 && ssv < 0x1p200 && fabs(alv) < 0x1p200 && smax < 0x1p800)) != 0) {
+    if (redo) {
       taken = true;
       if (PARTS > 1 && part != 0) return;
       slow(Vs, Ds, Zs, PARTS > 1 ? RT + 16 * (PARTS - 1) : nact > H ? RT : H, nb, tau);

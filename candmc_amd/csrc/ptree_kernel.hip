@@ -318,8 +318,9 @@ __device__ __forceinline__ void leaf16_tall_body(double* __restrict__ A, int64_t
     zero_below(Tl, b, strip, lane);
   }
   double* Vp = Vk + (S > 1 ? 16 * part : part - 1) * P16_TILE;   // this part's tiles of the panel
-  auto panel = [&](int k) {                       // another strip's panel: its columns, then V and T_kk are there
+  auto panel = [&](int k) {                       // another strip's panel: its columns and its check, then V and T_kk are there
     for (int j = 16 * k; j < min(b, 16 * k + 16); ++j) __syncthreads();
+    __syncthreads();
     __syncthreads();
   };
   // this part's share of V_kᵀ·(D; a) into X, for all parts after a barrier
