@@ -161,14 +161,15 @@ __device__ __forceinline__ void p16_fma_bc(double& acc, double z, double t) {
   asm("v_fmac_f64_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf" : "+&v"(acc) : "v"(z), "v"(t), "n"(C));
 }
 
-// sqrt and the two reciprocals of dlarfg for ss = ‖x‖² in (2^-200, 2^200)
-// and |alpha| < 2^200: beta = −sign(alpha)·sqrt(alpha² + ss) by the
+// sqrt and the two reciprocals of dlarfg for ss = ‖x‖² in (2^-960, 2^960)
+// and |alpha| < 2^480: beta = −sign(alpha)·sqrt(alpha² + ss) by the
 // Goldschmidt iteration from the hardware's reciprocal square root with two
-// residual corrections; no operand scaling is needed in this range.  ss = 0
+// residual corrections; no operand scaling is needed in this range (the
+// residual g² − x is a multiple of 2^-1064, and 1/beta at most 2^480).  ss = 0
 // stands for a zero x: H = I, beta = alpha and tau = 0, with scal and rb finite
 // (they meet zeros only).
 __device__ __forceinline__ void p16_larfg(double alpha, double ss, double& beta, double& tau, double& scal, double& rb) {
-  const double x = fmax(fma(alpha, alpha, ss), 0x1p-400);
+  const double x = fmax(fma(alpha, alpha, ss), 0x1p-960);
   const double y = __builtin_amdgcn_rsq(x);
   double g = x * y, h = 0.5 * y;
   const double r = fma(-h, g, 0.5);
@@ -221,7 +222,7 @@ struct Panel16 {
   static constexpr int H = PARTS > 1 ? RT : RT > 8 ? 8 : RT > 4 ? 4 : RT;
   double pr[P16];          // pivot rows
   double tau, scale;
-  double ssv, alv, smax;   // what decides the fast range: ‖x‖², alpha per column, largest |dot|
+  double ssv, alv;         // what decides the fast range: ‖x‖² and alpha per column
 
   // part ≠ 0, opaque as nact in column()
   __device__ __forceinline__ bool low() const {
@@ -305,7 +306,6 @@ struct Panel16 {
       pr[J] = c > J ? fma(-tj, wv, p) : (c == J ? beta : p);
       Zc[J * P16_LD] = wv * scale * -tj;        // four lanes, one value
     }
-    smax = fmax(smax, fabs(s));
     ssv = c == J ? s : ssv;
     alv = c == J ? p : alv;
     tau = c == J ? tj : tau;
@@ -424,7 +424,6 @@ struct Panel16 {
     tau = 0.0;
     scale = 1.0;
     ssv = alv = 1.0;
-    smax = 0.0;
     // the strip may come straight from MFMAs, whose results the inline VALU
     // code below must not read before they land
     __builtin_amdgcn_sched_barrier(0);
@@ -451,9 +450,11 @@ struct Panel16 {
     P16_STEP(0) P16_STEP(1) P16_STEP(2) P16_STEP(3) P16_STEP(4) P16_STEP(5) P16_STEP(6) P16_STEP(7)
     P16_STEP(8) P16_STEP(9) P16_STEP(10) P16_STEP(11) P16_STEP(12) P16_STEP(13) P16_STEP(14) P16_STEP(15)
 #undef P16_STEP
-    // the fast range: ‖x‖² in (2^-200, 2^200) or x = 0, |alpha| < 2^200, dots
-    // far from overflow; a NaN or infinity fails it
-    bool bad = !((ssv > 0x1p-200 && ssv < 0x1p200) || ssv == 0.0) || !(fabs(alv) < 0x1p200 && smax < 0x1p800);
+    // the fast range: ‖x‖² in (2^-960, 2^960) or x = 0, |alpha| < 2^480; a NaN
+    // or infinity fails it.  Dots of two columns in range stay below 2^960 and
+    // lose nothing to underflow that counts (2^-1074 against 2^-960); one that
+    // overflows makes its column infinite, which that column's own step shows.
+    bool bad = !((ssv > 0x1p-960 && ssv < 0x1p960) || ssv == 0.0) || !(fabs(alv) < 0x1p480);
     if (__builtin_amdgcn_ballot_w64(ssv == 0.0) != 0) {
       // really nothing there, or entries too small to square?  (they are as
       // their column's own step found them)

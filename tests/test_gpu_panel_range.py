@@ -89,3 +89,37 @@ def test_entries_too_small_to_square(Q, m, b, row):
     ref, rtau = O.local_tsqr(np.asfortranarray(A))
     assert np.abs(tau - rtau[:b]).max() < 64 * m * EPS
     assert np.abs(np.triu(YR[:b]) - np.triu(ref[:b])).max() < 64 * m * EPS * np.abs(ref).max()
+
+
+@pytest.mark.parametrize("e", [-470, -300, 300, 470])
+@pytest.mark.parametrize("m,b", LEAVES)
+def test_scaled_leaf(Q, m, b, e):
+    """A·2^e (entries 1e±141 and 1e±90) takes the same steps: the same
+    reflectors, R scaled exactly."""
+    A = O.gaussian(m, b, m + b)
+    YR, T, tau = leaf(Q, A)
+    YS, TS, ts = leaf(Q, np.ldexp(A, e))
+    assert np.array_equal(T, TS) and np.array_equal(tau, ts)
+    assert np.array_equal(np.tril(YR, -1), np.tril(YS, -1))
+    assert np.array_equal(np.ldexp(np.triu(YR[:b]), e), np.triu(YS[:b]))
+
+
+@pytest.mark.parametrize("e", [-470, 300])
+@pytest.mark.parametrize("m,b,P", [(512, 16, 4), (600, 64, 3), (1300, 128, 5), (2000, 100, 0)])
+def test_scaled_tree(Q, m, b, P, e):
+    A = O.gaussian(m, b, m + b)
+    assert np.array_equal(np.ldexp(tree_r(Q, A, P), e), tree_r(Q, np.ldexp(A, e), P))
+
+
+@pytest.mark.parametrize("m,b", [(256, 16), (256, 128), (512, 64)])
+def test_one_scaled_column(Q, m, b):
+    """A column of 1e±120 among ordinary ones: its own entries of R scaled, all
+    else the same."""
+    A = O.gaussian(m, b, m + b)
+    d = np.ones(b)
+    d[[3, b - 2]] = 2.0 ** -400, 2.0 ** 400
+    YR, T, tau = leaf(Q, A)
+    YS, TS, ts = leaf(Q, A * d)
+    assert np.array_equal(T, TS) and np.array_equal(tau, ts)
+    assert np.array_equal(np.tril(YR, -1), np.tril(YS, -1))
+    assert np.array_equal(np.triu(YR[:b]) * d, np.triu(YS[:b]))
