@@ -165,11 +165,9 @@ __device__ __forceinline__ void p16_fma_bc(double& acc, double z, double t) {
 // and |alpha| < 2^480: beta = −sign(alpha)·sqrt(alpha² + ss) by the
 // Goldschmidt iteration from the hardware's reciprocal square root with two
 // residual corrections; no operand scaling is needed in this range (the
-// residual g² − x is a multiple of 2^-1064, and 1/beta at most 2^480).  ss = 0
-// stands for a zero x: H = I, beta = alpha and tau = 0, with scal and rb finite
-// (they meet zeros only).
+// residual g² − x is a multiple of 2^-1064, and 1/beta at most 2^480).
 __device__ __forceinline__ void p16_larfg(double alpha, double ss, double& beta, double& tau, double& scal, double& rb) {
-  const double x = fmax(fma(alpha, alpha, ss), 0x1p-960);
+  const double x = fma(alpha, alpha, ss);
   const double y = __builtin_amdgcn_rsq(x);
   double g = x * y, h = 0.5 * y;
   const double r = fma(-h, g, 0.5);
@@ -177,13 +175,12 @@ __device__ __forceinline__ void p16_larfg(double alpha, double ss, double& beta,
   g = fma(g, r, g);
   g = fma(fma(-g, g, x), h, g);
   g = fma(fma(-g, g, x), h, g);
-  const double bt = -copysign(g, alpha);
-  // 1/bt from the refined reciprocal root h ≈ 1/(2g)
+  beta = -copysign(g, alpha);
+  // 1/beta from the refined reciprocal root h ≈ 1/(2g)
   double q = h + h;
   q = fma(q, fma(-g, q, 1.0), q);
-  rb = copysign(q, bt);
-  scal = recip_nr(alpha - bt);
-  beta = ss == 0.0 ? alpha : bt;
+  rb = copysign(q, beta);
+  scal = recip_nr(alpha - beta);
   tau = (beta - alpha) * rb;
 }
 
@@ -197,26 +194,31 @@ __device__ __forceinline__ void p16_larfg(double alpha, double ss, double& beta,
 //     reflector is [e_jj; x] and only row jj takes part (rows map as g + 4v).
 // LDS: Zs, a 16×16 tile whose row J receives −tau_J·v_qᵀv_J (q < J) and in
 // the end the panel's compact-WY T, transposed; Vs (RT tiles), where the
-// strip is kept for the slow path and the scaled vectors are left; Ds (one
+// strip is kept for slow() and the scaled vectors are left; Ds (one
 // tile), the pivot tile before and after.
 // With PARTS > 1 a leaf's panel is spread over as many waves, `part` of them
 // this one, all with RT tiles and one more, the pivot tile in part 0 and an
 // ordinary one in the others (its values then live in pr[0..3]; Ds is its
 // place in Vs).  Each part publishes its share of a column's dot products in
-// `ex` (two buffers of PARTS + 1 rows of sixteen, the last one the pivot row),
-// and after a workgroup barrier all of them form the same reflector.
+// `ex` (p16_ex_doubles: two buffers of PARTS + 1 rows of sixteen, the last one
+// the pivot row, then slow()'s), and after a workgroup barrier all of them form
+// the same reflector.  Other strips' waves meet these barriers by count; where
+// more of them follow (zero columns, slow()), the word p16_more of `ex` says so,
+// and ends at 0 for the barrier that publishes the panel.
 //
 // With GLOB (a leaf of one strip) nobody else reads the vectors: the tiles stay
-// in registers, scaled in place, and the slow path (`taken`) works on the leaf
-// in memory, which still holds the strip, and leaves the vectors there; col is
-// this lane's column, of `rows` rows (none past the matrix's last column).
+// in registers, scaled in place, and slow() works on the leaf in memory, which
+// still holds the strip; col is this part's first row of this lane's column, of
+// which it has `rows` rows (none past the matrix's last column).
+constexpr int p16_more(int parts) { return 2 * P16 * (parts + 1) + 2 * P16 * (2 * parts + 1); }   // (two words, taken in turn)
+constexpr int p16_ex_doubles(int parts) { return p16_more(parts) + 2; }
+
 template <int RT, bool NODE, int PARTS = 1, bool GLOB = false>
 struct Panel16 {
-  double* ex;
+  double* ex = nullptr;
   int part = 0;
-  double* col;
-  int rows;
-  bool taken = false;
+  double* col = nullptr;
+  int rows = 0;
   // the tiles [H, RT) are skipped as a whole once they are zero (never in a
   // tall leaf, whose parts stay full)
   static constexpr int H = PARTS > 1 ? RT : RT > 8 ? 8 : RT > 4 ? 4 : RT;
@@ -224,6 +226,13 @@ struct Panel16 {
   double tau, scale;
   double ssv, alv;         // what decides the fast range: ‖x‖² and alpha per column
 
+  // The fast range: ‖x‖² in (2^-960, 2^960) or x = 0, |alpha| < 2^480; a NaN
+  // or infinity fails it.  Dots of two columns in range stay below 2^960 and
+  // lose nothing to underflow that counts (2^-1074 against 2^-960); one that
+  // overflows makes its column infinite, which that column's own step shows.
+  __device__ static __forceinline__ bool in_range(double ss, double alpha) {
+    return ((ss > 0x1p-960 && ss < 0x1p960) || ss == 0.0) && fabs(alpha) < 0x1p480;
+  }
   // part ≠ 0, opaque as nact in column()
   __device__ __forceinline__ bool low() const {
     int p = part;
@@ -287,10 +296,13 @@ struct Panel16 {
       p = E[P16 * PARTS];
     }
     const double ss = readlane_d(s, J), alpha = readlane_d(p, J);
+    // a column without anything below its diagonal: H = I (by masks alone, as
+    // the values of p16_larfg then need not be numbers)
+    const int cj = (__double2loint(ss) | __double2hiint(ss)) != 0 ? J : P16;
     double beta, tj, scal, rb;
     p16_larfg(alpha, ss, beta, tj, scal, rb);
     const double wv = fma(scal, s, p);          // v_Jᵀ·(column c), v_J = [1; scal·x]
-    const double f = c > J ? wv * rb : 0.0;     // −tau·scal = 1/beta
+    const double f = c > cj ? wv * rb : 0.0;    // −tau·scal = 1/beta
     axpys<J, 0, H>(a, f);
     asm volatile("" : "+s"(nact));
     if constexpr (RT > H)
@@ -303,95 +315,209 @@ struct Panel16 {
         for (int q = 0; q + 4 <= N; q += 4) p16_axpyrows<J, 4>(pr + J + 1 + q, f);
         if constexpr (N % 4 != 0) p16_axpyrows<J, N % 4>(pr + P16 - N % 4, f);
       }
-      pr[J] = c > J ? fma(-tj, wv, p) : (c == J ? beta : p);
+      pr[J] = c > cj ? fma(-tj, wv, p) : (c == cj ? beta : p);
       Zc[J * P16_LD] = wv * scale * -tj;        // four lanes, one value
     }
     ssv = c == J ? s : ssv;
     alv = c == J ? p : alv;
-    tau = c == J ? tj : tau;
-    scale = c == J ? scal : scale;
+    tau = c == cj ? tj : tau;
+    scale = c == cj ? scal : scale;
   }
 
-  // The whole panel with dlarfg's general semantics (rescaling, zero and
-  // non-finite columns), in memory: nt tiles in Vs, the pivot tile in Ds.
-  __device__ __forceinline__ void slow(double* Vs, double* Ds, double* Zs, int nt, int nb, double& tau_out) const {
+  // The whole panel again with dlarfg's general semantics (norms that have to
+  // be rescaled, non-finite columns), on this part's copy: nt tiles in Vs (GLOB:
+  // the leaf in memory), the pivot tile in Ds; one column at a time with the
+  // updates masked to the columns behind it.  A column of very large or small
+  // entries is first scaled by a power of two, which leaves its reflector as it
+  // is and brings data of any common size into the range of p16_larfg; what is
+  // left (entries too far apart, NaN, infinities) takes up to three more passes
+  // and dlarfg_scalar.  Two passes a column, two or four tiles in flight; keeping
+  // the strip in the registers that are free here spilled in the straight-line
+  // steps.  hh_recon_qr with every entry around 1e-200: 256×16 130 µs (78 in
+  // range), 32768×128 1220 (498), 65536×16 480 (187); with one value in
+  // flight, a division an element and one wave for a whole tall leaf 372, 3600 and
+  // 4470.
+  __device__ __forceinline__ double slow(double* Vs, double* Ds, double* Zs, int nt, int nb, int& bar) const {
     const int lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
+    const bool first = PARTS == 1 || part == 0;   // holds the pivot tile
+    asm volatile("" : "+s"(nt));                  // (a count the loops do not unroll by)
     auto sync = []() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup"); };
-    // element v of this lane's column in tile t (t < 0: the pivot tile)
-    auto place = [&](int t, int v) -> double* {
-      if (GLOB && t >= 0) {
-        const int row = 16 * (t + 1) + 4 * g + v;
-        return row < rows ? col + row : nullptr;
+    auto load = [&](int t) {                      // this lane's column in tile t
+      if constexpr (GLOB) return p16_rows_load(col + 16 * (t + 1) + 4 * g, rows - 16 * (t + 1) - 4 * g, rows > 0);
+      else return p16_load(Vs + t * P16_TILE, lane);
+    };
+    auto load_j = [&](int t, int j) {             // column j there
+      if constexpr (GLOB) {
+        const double* q = reinterpret_cast<const double*>(__double_as_longlong(
+            readlane_d(__longlong_as_double(reinterpret_cast<uintptr_t>(col)), j)));
+        const int left = __builtin_amdgcn_readlane(rows, j) - 16 * (t + 1) - 4 * g;
+        return p16_rows_load(q + 16 * (t + 1) + 4 * g, left, true);
+      } else {
+        return p16_load(Vs + t * P16_TILE, (lane & 48) | j);
       }
-      return (t < 0 ? Ds : Vs + t * P16_TILE) + (g + 4 * v) * P16_LD + c;
     };
-    auto at = [&](int t, int v) {
-      const double* q = place(t, v);
-      return !GLOB || q ? *q : 0.0;
+    auto store = [&](int t, const dbl4& x) {
+      if constexpr (GLOB) p16_rows_store(col + 16 * (t + 1) + 4 * g, x, rows - 16 * (t + 1) - 4 * g, rows > 0);
+      else p16_store(Vs + t * P16_TILE, x, lane);
     };
-    auto put = [&](int t, int v, double x) {
-      double* q = place(t, v);
-      if (!GLOB || q) *q = x;
+    // f(t, x_t) for all tiles, CH of them loaded at a time
+    constexpr int CH = PARTS > 1 ? 4 : 2;
+    auto each = [&](auto get, auto f) {
+#pragma unroll 1
+      for (int t = 0; t < nt; t += CH) {
+        decltype(get(0)) x[CH];
+#pragma unroll
+        for (int i = 0; i < CH; ++i) x[i] = get(min(t + i, nt - 1));
+#pragma unroll
+        for (int i = 0; i < CH; ++i)
+          if (t + i < nt) f(t + i, x[i]);
+      }
     };
-    auto pivot_row = [&](int v) { return NODE ? g + 4 * v : 4 * g + v; };
-    const int t0 = NODE ? 0 : -1;
-    double tau = 0.0;
+    struct Two {
+      dbl4 j, c;
+    };
+    auto both = [&](int j) { return [&, j](int t) { return Two{load_j(t, j), load(t)}; }; };
+    auto top = [](const dbl4& x) { return fmax(fmax(fabs(x[0]), fabs(x[1])), fmax(fabs(x[2]), fabs(x[3]))); };
+    auto rows_max = [](double m) {
+      m = fmax(m, __shfl_xor(m, 16));
+      return fmax(m, __shfl_xor(m, 32));
+    };
+    auto ldexp4 = [](const dbl4& x, int e) { return dbl4{ldexp(x[0], e), ldexp(x[1], e), ldexp(x[2], e), ldexp(x[3], e)}; };
+    // the values of the pivot tile (or of a low part's first one) below the
+    // diagonal of column j, which belong to a leaf's vectors
+    auto low_row = [&](int v, int j) { return !NODE && (!first || 4 * g + v > j); };
+    auto below = [&](const dbl4& x, int j) {
+      dbl4 y;
+#pragma unroll
+      for (int v = 0; v < 4; ++v) y[v] = low_row(v, j) ? x[v] : 0.0;
+      return y;
+    };
+    // sums and largest values over all parts, and the pivot part's q
+    auto exchange = [&](double& sum, double& m, double& q) {
+      if constexpr (PARTS > 1) {
+        double* E = ex + 2 * P16 * (PARTS + 1) + (bar & 1) * (P16 * (2 * PARTS + 1)) + c;
+        E[P16 * part] = sum;
+        E[P16 * (PARTS + part)] = m;
+        if (first) {
+          E[P16 * 2 * PARTS] = q;
+          if (lane == 0) ex[p16_more(PARTS) + (bar & 1)] = 1.0;
+        }
+        __syncthreads();
+        sum = E[0];
+        m = E[P16 * PARTS];
+#pragma unroll
+        for (int i = 1; i < PARTS; ++i) {
+          sum += E[P16 * i];
+          m = fmax(m, E[P16 * (PARTS + i)]);
+        }
+        q = E[P16 * 2 * PARTS];
+        ++bar;
+      }
+    };
+    double none = 0.0, zero = 0.0;
+
+    double mx = top(p16_load(Ds, lane));
+    each(load, [&](int, const dbl4& x) { mx = fmax(mx, top(x)); });
+    mx = rows_max(mx);
+    exchange(zero, mx, none);
+    int e = mx > 0.0 && mx < INFINITY ? __builtin_amdgcn_frexp_exp(mx) : 0;
+    if (abs(e) < 400) e = 0;
+    if (__builtin_amdgcn_ballot_w64(e != 0) != 0) {
+      p16_store(Ds, ldexp4(p16_load(Ds, lane), -e), lane);
+      each(load, [&](int t, const dbl4& x) { store(t, ldexp4(x, -e)); });
+    }
+    double tl = 0.0, scale = 1.0;
+    sync();
 #pragma unroll 1
     for (int j = 0; j < nb; ++j) {
-      const int src = (lane & 48) | j;
       const int jr = trow_of(j);
-      const double p = Ds[jr * P16_LD + c];
-      const double alpha = readlane_d(p, j);
-      auto below = [&](int t, int v) { return t >= 0 || pivot_row(v) > j; };
-      double mx = 0.0;
-#pragma unroll 1
-      for (int t = t0; t < nt; ++t)
-        for (int v = 0; v < 4; ++v)
-          if (below(t, v)) mx = fmax(mx, fabs(at(t, v)));
-      mx = fmax(mx, __shfl_xor(mx, 16));
-      mx = readlane_d(fmax(mx, __shfl_xor(mx, 32)), j);
-      double s2 = 0.0;
-#pragma unroll 1
-      for (int t = t0; t < nt; ++t)
-        for (int v = 0; v < 4; ++v)
-          if (below(t, v)) {
-            const double x = at(t, v) / mx;
-            s2 += x * x;
-          }
-      s2 = readlane_d(xr_cross_rows(s2), j);
-      const Reflector h = dlarfg_scalar(alpha, mx == 0.0 ? 0.0 : mx * sqrt(s2));
-      if (c == j && h.tau != 0.0)
-  #pragma unroll 1
-      for (int t = t0; t < nt; ++t)
-          for (int v = 0; v < 4; ++v)
-            if (below(t, v)) {
-              double x = at(t, v);
+      double p = Ds[jr * P16_LD + c];             // (a low part's is not used)
+      auto dots = [&](double& m) {
+        const dbl4 xd = below(p16_load(Ds, (lane & 48) | j), j), d = below(p16_load(Ds, lane), j);
+        dbl4 s = xd * d;
+        m = top(d);
+        each(both(j), [&](int, const Two& x) {
+          s += x.j * x.c;
+          m = fmax(m, top(x.c));
+        });
+        m = rows_max(m);
+        return xr_cross_rows((s[0] + s[1]) + (s[2] + s[3]));
+      };
+      double m, s = dots(m);
+      exchange(s, m, p);
+      const double ss = readlane_d(s, j), alpha = readlane_d(p, j);
+      m = readlane_d(m, j);
+      double beta, tj, fs, sc, wv;                // sc: the vector's scale, fs: the update's factor
+      if (ss != 0.0 && in_range(ss, alpha)) {
+        p16_larfg(alpha, ss, beta, tj, sc, fs);
+        wv = fma(sc, s, p);
+      } else {
+        double xnorm = m == 0.0 ? 0.0 : NAN;      // (a NaN beside entries that are none)
+        if (m > 0.0 && m < INFINITY && ss == ss) {
+          const int em = __builtin_amdgcn_frexp_exp(m);
+          dbl4 q = ldexp4(below(p16_load(Ds, lane), j), -em);
+          q *= q;
+          each(load, [&](int, const dbl4& x) {
+            const dbl4 y = ldexp4(x, -em);
+            q += y * y;
+          });
+          double n2 = xr_cross_rows((q[0] + q[1]) + (q[2] + q[3]));
+          exchange(n2, zero, none);
+          xnorm = ldexp(sqrt(readlane_d(n2, j)), em);
+        }
+        const Reflector h = dlarfg_scalar(alpha, xnorm);
+        if (h.tau != 0.0) {
+          if (c == j) {
+            auto vec = [&](dbl4 x) {
               for (int k = 0; k < h.knt; ++k) x *= 0x1p969;
-              put(t, v, x * h.scal);
-            }
-      sync();
-      double s = 0.0;
+              return x * h.scal;
+            };
+            const dbl4 d = p16_load(Ds, lane), y = vec(d);
+            dbl4 z;
+#pragma unroll
+            for (int v = 0; v < 4; ++v) z[v] = low_row(v, j) ? y[v] : d[v];
+            p16_store(Ds, z, lane);
 #pragma unroll 1
-      for (int t = t0; t < nt; ++t)
-        for (int v = 0; v < 4; ++v) {
-          const double x = __shfl(at(t, v), src);
-          if (below(t, v)) s += x * at(t, v);
+            for (int t = 0; t < nt; ++t) store(t, vec(load(t)));
+          }
+          sync();
+          s = dots(m);
+          exchange(s, m, p);
         }
-      const double wv = p + xr_cross_rows(s), f = h.tau * wv;
-#pragma unroll 1
-      for (int t = t0; t < nt; ++t)
-        for (int v = 0; v < 4; ++v) {
-          const double x = __shfl(at(t, v), src);
-          if (c > j && below(t, v)) put(t, v, at(t, v) - f * x);
-        }
-      if (g == 0) {
-        Ds[jr * P16_LD + c] = c > j ? p - f : (c == j ? h.beta : p);
-        Zs[j * P16_LD + c] = c < j ? -h.tau * wv : 0.0;
+        wv = p + s;
+        beta = h.beta;
+        tj = h.tau;
+        fs = -h.tau;
+        sc = 1.0;
       }
-      if (c == j) tau = h.tau;
+      if (c > j) {
+        const double f = wv * fs;
+        const dbl4 xd = p16_load(Ds, (lane & 48) | j), d = p16_load(Ds, lane);
+        dbl4 z;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) z[v] = low_row(v, j) ? fma(xd[v], f, d[v]) : d[v];
+        p16_store(Ds, z, lane);
+        each(both(j), [&](int t, const Two& x) { store(t, x.j * f + x.c); });
+      }
+      sync();
+      if (first && g == 0) {
+        Ds[jr * P16_LD + c] = c > j ? fma(-tj, wv, p) : (c == j ? beta : p);
+        Zs[j * P16_LD + c] = c < j ? wv * scale * -tj : 0.0;
+      }
+      if (c == j) {
+        tl = tj;
+        scale = sc;
+      }
       sync();
     }
-    tau_out = tau;
+    const dbl4 d = p16_load(Ds, lane);
+    dbl4 z;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) z[v] = low_row(v, c) ? d[v] * scale : ldexp(d[v], e);
+    p16_store(Ds, z, lane);
+    each(load, [&](int t, const dbl4& x) { store(t, x * scale); });
+    sync();
+    return tl;
   }
 
   template <int J, int Q = 0>
@@ -429,7 +555,7 @@ struct Panel16 {
     __builtin_amdgcn_sched_barrier(0);
     asm volatile("s_nop 15\n s_nop 15\n s_nop 15");
     __builtin_amdgcn_sched_barrier(0);
-    // kept for the slow path: straight-line columns with one test at the end
+    // kept for slow(): straight-line columns with one test at the end
     // cost less than a way out of every column
     p16_store(Ds, D, lane);
     if constexpr (!GLOB)
@@ -450,12 +576,9 @@ struct Panel16 {
     P16_STEP(0) P16_STEP(1) P16_STEP(2) P16_STEP(3) P16_STEP(4) P16_STEP(5) P16_STEP(6) P16_STEP(7)
     P16_STEP(8) P16_STEP(9) P16_STEP(10) P16_STEP(11) P16_STEP(12) P16_STEP(13) P16_STEP(14) P16_STEP(15)
 #undef P16_STEP
-    // the fast range: ‖x‖² in (2^-960, 2^960) or x = 0, |alpha| < 2^480; a NaN
-    // or infinity fails it.  Dots of two columns in range stay below 2^960 and
-    // lose nothing to underflow that counts (2^-1074 against 2^-960); one that
-    // overflows makes its column infinite, which that column's own step shows.
-    bool bad = !((ssv > 0x1p-960 && ssv < 0x1p960) || ssv == 0.0) || !(fabs(alv) < 0x1p480);
-    if (__builtin_amdgcn_ballot_w64(ssv == 0.0) != 0) {
+    int bar = 0;
+    bool redo = __builtin_amdgcn_ballot_w64(!in_range(ssv, alv)) != 0;
+    if (const uint64_t z = __builtin_amdgcn_ballot_w64(ssv == 0.0)) {
       // really nothing there, or entries too small to square?  (they are as
       // their column's own step found them)
       double nz = 0.0;
@@ -466,25 +589,35 @@ struct Panel16 {
       if (!NODE)
 #pragma unroll
         for (int q = 0; q < P16; ++q) nz = fmax(nz, (PARTS > 1 && part != 0 ? q < 4 : q > c) ? fabs(pr[q]) : 0.0);
-      bad |= ssv == 0.0 && nz > 0.0;
-    }
-    bool redo = __builtin_amdgcn_ballot_w64(bad) != 0;
-    if constexpr (PARTS > 1) {                    // one decision for all parts
-      double* E = ex + (nb & 1) * (P16 * (PARTS + 1));
-      if (lane == 0) E[part] = redo ? 1.0 : 0.0;
-      __syncthreads();
-      redo = false;
+      bool some = __builtin_amdgcn_ballot_w64(ssv == 0.0 && nz > 0.0) != 0;
+      if constexpr (PARTS > 1) {                  // one decision for all parts
+        double* E = ex + 2 * P16 * (PARTS + 1);
+        if (lane == 0) {
+          E[part] = some ? 1.0 : 0.0;
+          if (part == 0) ex[p16_more(PARTS)] = 1.0;
+        }
+        __syncthreads();
+        some = false;
 #pragma unroll
-      for (int q = 0; q < PARTS; ++q) redo |= E[q] != 0.0;
-      redo = __builtin_amdgcn_readfirstlane(redo) != 0;
+        for (int q = 0; q < PARTS; ++q) some |= E[q] != 0.0;
+        some = __builtin_amdgcn_readfirstlane(some) != 0;
+        bar = 1;
+      }
+      redo |= some;
+      if (PARTS == 1 || part == 0)
+        for (int q = 0; q < P16; ++q)
+          if (z >> q & 1) Zc[q * P16_LD] = 0.0;
     }
-    if constexpr (GLOB)   // (without meaning on the slow path)
+    if constexpr (GLOB)   // (without meaning if the panel is redone)
 #pragma unroll
       for (int t = 0; t < RT; ++t) a[t] *= scale;
-    if (redo) {
-      taken = true;
+    if (__builtin_expect(redo, 0)) {
+      tau = slow(Vs, Ds, Zs, nact > H ? RT : H, nb, bar);
+      if constexpr (GLOB)
+#pragma unroll
+        for (int t = 0; t < RT; ++t)
+          a[t] = p16_rows_load(col + 16 * (t + 1) + 4 * (lane >> 4), rows - 16 * (t + 1) - 4 * (lane >> 4), rows > 0);
       if (PARTS > 1 && part != 0) return;
-      slow(Vs, Ds, Zs, PARTS > 1 ? RT + 16 * (PARTS - 1) : nact > H ? RT : H, nb, tau);
     } else {
       if constexpr (!GLOB)
 #pragma unroll
@@ -497,6 +630,7 @@ struct Panel16 {
 #pragma unroll
       for (int q = 0; q < P16; ++q) Ds[trow_of(q) * P16_LD + c] = !NODE && q > c ? pr[q] * scale : pr[q];
     }
+    if (PARTS > 1 && lane == 0) ex[p16_more(PARTS) + (bar & 1)] = 0.0;
     D = p16_load(Ds, lane);
     double z[P16], trow[P16];
 #pragma unroll

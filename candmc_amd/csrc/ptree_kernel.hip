@@ -259,7 +259,7 @@ __device__ __forceinline__ void leaf16_body(double* __restrict__ A, int64_t lda,
 // ---------------------------------------------------------------------------
 template <int S, int P>
 constexpr int tall_smem_doubles() {
-  return ((S > 1 ? 16 * P : P - 1) + S * (S + 1) / 2 + 1 + (S - 1) * P) * P16_TILE + 2 * P16 * (P + 1);
+  return ((S > 1 ? 16 * P : P - 1) + S * (S + 1) / 2 + 1 + (S - 1) * P) * P16_TILE + p16_ex_doubles(P);
 }
 
 template <int S, int P>
@@ -318,10 +318,11 @@ __device__ __forceinline__ void leaf16_tall_body(double* __restrict__ A, int64_t
     zero_below(Tl, b, strip, lane);
   }
   double* Vp = Vk + (S > 1 ? 16 * part : part - 1) * P16_TILE;   // this part's tiles of the panel
-  auto panel = [&](int k) {                       // another strip's panel: its columns and its check, then V and T_kk are there
+  auto panel = [&](int k) {                       // another strip's panel: its columns, then V and T_kk are there
     for (int j = 16 * k; j < min(b, 16 * k + 16); ++j) __syncthreads();
-    __syncthreads();
-    __syncthreads();
+    int bar = 0;
+    do __syncthreads();
+    while (ex[p16_more(P) + (bar++ & 1)] != 0.0);
   };
   // this part's share of V_kᵀ·(D; a) into X, for all parts after a barrier
   auto share = [&](int k) {
@@ -368,13 +369,12 @@ __device__ __forceinline__ void leaf16_tall_body(double* __restrict__ A, int64_t
     __syncthreads();
   }
   if (strip >= nblk) return;                      // (no barrier is left)
-  bool taken = false;                             // the vectors are in memory already
   {
     const int k = strip;
     __builtin_amdgcn_s_setprio(3);
     Panel16<NB, false, P, S == 1> F;
     F.col = Ac - 4 * g;
-    F.rows = colok ? r : 0;
+    F.rows = colok ? r - 256 * part : 0;
     F.ex = ex;
     F.part = part;
     F.factor(D, a, NB, min(P16, b - 16 * k), lane, Ts + p16_slot(k, k), Vp + P16_TILE,
@@ -399,7 +399,6 @@ __device__ __forceinline__ void leaf16_tall_body(double* __restrict__ A, int64_t
       for (int t = 0; t < NB; ++t) a[t] = p16_load(Vp + (t + 1) * P16_TILE, lane);
     } else {
       if (part != 0) D = p16_load(Vp, lane);
-      taken = F.taken;
     }
     finish(k);
     __syncthreads();
@@ -426,13 +425,11 @@ __device__ __forceinline__ void leaf16_tall_body(double* __restrict__ A, int64_t
     put_t_tile(Tl, b, strip, nblk - 1, p16_tcol(Ts, strip, nblk - 1, lane), lane);
   }
   // the rows below the last panel's block
-  if (!taken) {
-    const int t0 = part == 0 ? nblk : 0;
-    p16_rows_store(Ac + 16 * t0, D, rg - 16 * t0, colok);
+  const int t0 = part == 0 ? nblk : 0;
+  p16_rows_store(Ac + 16 * t0, D, rg - 16 * t0, colok);
 #pragma unroll
-    for (int t = 0; t < NB; ++t)
-      if (t0 + t + 1 < 16) p16_rows_store(Ac + 16 * (t0 + t + 1), a[t], rg - 16 * (t0 + t + 1), colok);
-  }
+  for (int t = 0; t < NB; ++t)
+    if (t0 + t + 1 < 16) p16_rows_store(Ac + 16 * (t0 + t + 1), a[t], rg - 16 * (t0 + t + 1), colok);
 }
 
 // ---------------------------------------------------------------------------

@@ -123,3 +123,36 @@ def test_one_scaled_column(Q, m, b):
     assert np.array_equal(T, TS) and np.array_equal(tau, ts)
     assert np.array_equal(np.tril(YR, -1), np.tril(YS, -1))
     assert np.array_equal(np.triu(YR[:b]) * d, np.triu(YS[:b]))
+
+
+@pytest.mark.parametrize("m,b", [(256, 16), (65536, 16), (8192, 64), (32768, 128)])
+@pytest.mark.parametrize("kind", ["1e-200", "1e200", "nan"])
+def test_general_route_is_not_much_slower(Q, m, b, kind):
+    """Panels that have to be redone column by column: at most four times an
+    ordinary panel's time (three to five passes over a strip in place of two,
+    serial loads in place of none; through memory it was five to twenty-four)."""
+    print("general route", m, b, kind, flush=True)
+    A = Q.to_gpu(O.gaussian(m, b, m + b))
+    Z = A.clone()
+    if kind == "nan":
+        Z[5 * m + 7] = float("nan")
+    else:
+        Z *= float(kind)
+    W = torch.zeros(b * b, dtype=torch.float64, device="cuda")
+    work = torch.empty_like(A)
+
+    def us(src):
+        ev = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+        ts = []
+        for _ in range(9):
+            work.copy_(src)
+            torch.cuda.synchronize()
+            ev[0].record()
+            Q.hh_recon_qr(work, m, m, b, W, numPes=0, sync=False)
+            ev[1].record()
+            torch.cuda.synchronize()
+            ts.append(ev[0].elapsed_time(ev[1]))
+        return sorted(ts)[4]
+
+    us(A)
+    assert us(Z) < 4 * us(A)
