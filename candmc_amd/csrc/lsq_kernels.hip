@@ -428,16 +428,22 @@ trsm_chain_kernel(const double* __restrict__ R, int64_t ldr, int64_t n, const do
         x[i][v] = row < bp && c < nr ? load_coherent(Bc + jp + row) : 0.0;
       }
 #pragma unroll
-    for (int i = 0; i < 2; ++i) p16_store(xs + row_of(i) * P16_TILE, -x[i], lane);
+    for (int i = 0; i < 2; ++i) p16_store(xs + row_of(i) * P16_TILE, x[i], lane);
     __syncthreads();
+    // the block's product by itself, in two chains, and one subtraction: summed
+    // onto y it would round 128 times at y's size
+    dbl4 s[2][2] = {{zero, zero}, {zero, zero}};
 #pragma unroll
     for (int kt = 0; kt < 8; ++kt) {
       const dbl4 xk = p16_load(xs + kt * P16_TILE, lane);
 #pragma unroll
       for (int v = 0; v < 4; ++v)
 #pragma unroll
-        for (int i = 0; i < 2; ++i) y[i] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[i][kt][v], xk[v], y[i], 0, 0, 0);
+        for (int i = 0; i < 2; ++i)
+          s[i][kt >> 2] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[i][kt][v], xk[v], s[i][kt >> 2], 0, 0, 0);
     }
+#pragma unroll
+    for (int i = 0; i < 2; ++i) y[i] -= s[i][0] + s[i][1];
     if (d + 1 < ndep) load_block(d + 1);   // in flight during the next wait
   }
 #pragma unroll

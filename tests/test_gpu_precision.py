@@ -1,0 +1,62 @@
+"""GPU tests of accuracy: the error of the FP64 products, factorizations and
+solves against the same thing in extended precision, next to the error of a
+plain FP64 numpy rendering of the same algorithm on the same inputs.  Both are
+rounding errors of a few units; the bound is a small multiple of numpy's, the
+mean over several seeds (sums that start from a large value, or long chains of
+them, show as more)."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+X = np.longdouble
+SEEDS = range(6)
+
+
+@pytest.fixture(scope="module")
+def Q():
+    from candmc_amd import qr
+    assert torch.cuda.is_available(), "GPU tests need an MI355X"
+    return qr
+
+
+def rnd(m, n, seed):
+    return np.asfortranarray(np.random.default_rng(seed).standard_normal((m, n)))
+
+
+def err(got, ref):
+    e = (got - ref).astype(np.float64)
+    return float(np.linalg.norm(e) / np.linalg.norm(ref.astype(np.float64)))
+
+
+def zeros(n):
+    return torch.zeros(n, dtype=torch.float64, device="cuda")
+
+
+@pytest.mark.parametrize("n,nr", [(512, 3), (600, 1), (600, 16), (1100, 5)])
+@pytest.mark.parametrize("trans", [False, True])
+def test_triangular_solve(Q, n, nr, trans):
+    """The chained solve (four blocks of 128 rows and more): at most twice the
+    error of the same block steps in numpy (block inverse, product, subtraction)."""
+    ours, plain = [], []
+    for seed in SEEDS:
+        R = np.triu(rnd(n, n, seed)) / np.sqrt(n) + 2 * np.diag(np.sign(rnd(n, 1, seed + 50)[:, 0]))
+        B = rnd(n, nr, seed + 100)
+        M = R.T if trans else R
+        ref = B.astype(X)
+        for i in (range(n) if trans else range(n - 1, -1, -1)):
+            ref[i] /= X(M[i, i])
+            rest = slice(i + 1, n) if trans else slice(0, i)
+            ref[rest] -= np.outer(M[rest, i].astype(X), ref[i])
+        Y = B.copy()
+        blocks = [(j, min(n, j + 128)) for j in range(0, n, 128)]
+        for a, b in (blocks if trans else blocks[::-1]):
+            Y[a:b] = np.linalg.inv(M[a:b, a:b]) @ Y[a:b]
+            rest = slice(b, n) if trans else slice(0, a)
+            Y[rest] -= M[rest, a:b] @ Y[a:b]
+        plain.append(err(Y, ref))
+        print("trsm", n, nr, trans, seed, flush=True)
+        dR, dB = Q.to_gpu(np.asfortranarray(R)), Q.to_gpu(B)
+        Q.trsm_r(dR, n, n, dB, n, nr, trans=trans)
+        ours.append(err(Q.from_gpu(dB, n, nr), ref))
+    assert np.mean(ours) < 2 * np.mean(plain), (np.mean(ours), np.mean(plain))
