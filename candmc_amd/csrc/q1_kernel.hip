@@ -312,7 +312,7 @@ q1_kernel(const double* __restrict__ nodeV2, const double* __restrict__ nodeT, c
   const int nrow = (ml + 15) / 16;
   auto row_product = [&](int t, dbl4 (&x)[8]) {
     const dbl4 zero = {0.0, 0.0, 0.0, 0.0};
-    dbl4 h0 = t <= hi ? get(S0, 0, t) : zero, l0 = two && t <= lo ? get(S0, 1, t) : zero, h1 = zero;
+    dbl4 h0 = zero, h1 = zero, l0 = zero;
 #pragma unroll
     for (int kt = 0; kt < 8; ++kt)
       if (kt <= hi && kt <= t) {
@@ -332,7 +332,11 @@ q1_kernel(const double* __restrict__ nodeV2, const double* __restrict__ nodeT, c
             l0 = __builtin_amdgcn_mfma_f64_16x16x4f64(a, x[kt][v], l0, 0, 0, 0);
           }
       }
+    // C_l last: summed onto it (a value near 1 on the diagonal) the product
+    // would round at its size in every step
     h0 += h1;
+    if (t <= hi) h0 += get(S0, 0, t);
+    if (two && t <= lo) l0 += get(S0, 1, t);
     const int row = 16 * t + tr;
     if (row < ml)
 #pragma unroll

@@ -60,3 +60,24 @@ def test_triangular_solve(Q, n, nr, trans):
         Q.trsm_r(dR, n, n, dB, n, nr, trans=trans)
         ours.append(err(Q.from_gpu(dB, n, nr), ref))
     assert np.mean(ours) < 2 * np.mean(plain), (np.mean(ours), np.mean(plain))
+
+
+@pytest.mark.parametrize("m,b", [(256, 32), (256, 128), (130, 100), (500, 64), (1000, 16)])
+def test_explicit_q(Q, m, b):
+    """construct_Q1 of one leaf from its own V and T, Q1 = [I; 0] − V·(T·V_topᵀ):
+    the largest error at most twice that of the same products in numpy."""
+    assert Q.plan_tsqr(m, b, 1)[0] == 1
+    ours, plain = [], []
+    for seed in SEEDS:
+        print("construct_Q1", m, b, seed, flush=True)
+        dA, R, tau, Q1 = Q.to_gpu(rnd(m, b, seed)), zeros(b * b), zeros(b), zeros(m * b)
+        td = zeros(Q.tree_data_size(m, b, 1))
+        Q.bitree_tsqr(dA, m, R, tau, m, b, numPes=1, output_Y=1, tree_data=td)
+        Q.construct_Q1(dA, m, tau, Q1, m, m, b, b, numPes=1, tree_data=td)
+        V = np.tril(Q.from_gpu(dA, m, b), -1) + np.eye(m, b)
+        T = np.triu(Q.from_gpu(td[:b * b], b, b))
+        E = np.eye(m, b)
+        ref = E - V.astype(X) @ (T.astype(X) @ V[:b].T.astype(X))
+        ours.append(float(abs(Q.from_gpu(Q1, m, b) - ref).max()))
+        plain.append(float(abs(E - V @ (T @ V[:b].T) - ref).max()))
+    assert np.mean(ours) < 2 * np.mean(plain), (np.mean(ours), np.mean(plain))
