@@ -66,16 +66,18 @@ __device__ __forceinline__ dbl4 ht_mmt(const double* X, const dbl4& y, dbl4 acc,
   for (int v = 0; v < 4; ++v) acc = __builtin_amdgcn_mfma_f64_16x16x4f64(p[v * P16_LD], y[v], acc, 0, 0, 0);
   return acc;
 }
-// acc + X·y for the unit lower triangle of X (what lies above it is other data)
-__device__ __forceinline__ dbl4 ht_mm_unit(const double* X, const dbl4& y, dbl4 acc, int lane) {
+// X·y for the unit lower triangle of X (what lies on and above its diagonal is
+// other data): y added to the strict triangle's product
+__device__ __forceinline__ dbl4 ht_mm_unit(const double* X, const dbl4& y, int lane) {
   const int r = perm16(lane & 15), k0 = 4 * (lane >> 4);
   const double* p = X + r * P16_LD + k0;
+  dbl4 acc = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
   for (int v = 0; v < 4; ++v) {
-    const double x = p[v], m = r > k0 + v ? x : (r == k0 + v ? 1.0 : 0.0);
-    acc = __builtin_amdgcn_mfma_f64_16x16x4f64(m, y[v], acc, 0, 0, 0);
+    const double x = p[v];
+    acc = __builtin_amdgcn_mfma_f64_16x16x4f64(r > k0 + v ? x : 0.0, y[v], acc, 0, 0, 0);
   }
-  return acc;
+  return acc + y;
 }
 
 // One panel of the signed LU: RT tiles below the diagonal tile, whose rows
@@ -288,11 +290,11 @@ __device__ __forceinline__ void lu16(const double* src, int64_t ld, double* smem
     __syncthreads();
     auto apply = [&]() {
       const dbl4 zero = {0.0, 0.0, 0.0, 0.0};
-      const dbl4 u = ht_mm_unit(LI + k * HT, D, zero, lane);
+      const dbl4 u = ht_mm_unit(LI + k * HT, D, lane);
       ht_store(hr_tile<W>(smem, k, s), u, lane);
 #pragma unroll
       for (int t = 0; t < RT; ++t)
-        if (t < nact) a[t] = ht_mm(hr_tile<W>(smem, k + 1 + t, k), -u, a[t], lane);
+        if (t < nact) a[t] -= ht_mm(hr_tile<W>(smem, k + 1 + t, k), u, zero, lane);
     };
     if (k + 1 < n) {   // the next strip first, alone (see leaf16_body)
       if (s == k + 1) apply();
@@ -401,7 +403,7 @@ __device__ __forceinline__ void hr16_body(const HrArgs& h, double* smem) {
           dbl4 acc = zero;
 #pragma unroll
           for (int e = 0; e < d; ++e) acc = ht_mm(hr_tile<W>(smem, s + d, s + e), x[e], acc, lane);
-          x[d] = -ht_mm_unit(LI + (s + d) * HT, acc, zero, lane);
+          x[d] = -ht_mm_unit(LI + (s + d) * HT, acc, lane);
         }
     }
     if (h.Uinv) {
@@ -472,7 +474,7 @@ __device__ __forceinline__ void hr16_body(const HrArgs& h, double* smem) {
 #pragma unroll
       for (int d = 0; d < W; ++d)
         if (s + d < n) {
-          dbl4 acc = ht_mm_unit(LI + (s + d) * HT, wt[d], zero, lane);
+          dbl4 acc = ht_mm_unit(LI + (s + d) * HT, wt[d], lane);
 #pragma unroll
           for (int e = 0; e < d; ++e) acc = ht_mm(hr_tile<W>(smem, s + d, s + e), wt[e], acc, lane);
           tt[d] = -acc;

@@ -81,3 +81,31 @@ def test_explicit_q(Q, m, b):
         ours.append(float(abs(Q.from_gpu(Q1, m, b) - ref).max()))
         plain.append(float(abs(E - V @ (T @ V[:b].T) - ref).max()))
     assert np.mean(ours) < 2 * np.mean(plain), (np.mean(ours), np.mean(plain))
+
+
+@pytest.mark.parametrize("b", [32, 64, 128])
+def test_signed_lu(Q, b):
+    """L and U of the signed LU of an orthonormal block against plain
+    right-looking elimination in numpy, which rounds an entry at every column
+    before it; here the sixteen columns of a strip are one update, which at two
+    strips already saves a third of an entry's roundings."""
+    ours, plain = [], []
+    for seed in SEEDS:
+        print("signed LU", b, seed, flush=True)
+        A = np.asfortranarray(np.linalg.qr(rnd(512, b, seed))[0][:b])
+
+        def lu(M):
+            for j in range(b):
+                M[j, j] -= -1 if M[j, j] > 0 else 1
+                M[j + 1:, j] /= M[j, j]
+                M[j + 1:, j + 1:] -= np.outer(M[j + 1:, j], M[j, j + 1:])
+            return M
+
+        ref, P = lu(A.astype(X)), lu(A.copy())
+        dA, R = Q.to_gpu(A), zeros(b * b)
+        Q.signed_NLU(dA, R, b, b, b)
+        G = Q.from_gpu(dA, b, b)
+        ours.append([err(np.triu(G), np.triu(ref)), err(np.tril(G, -1), np.tril(ref, -1))])
+        plain.append([err(np.triu(P), np.triu(ref)), err(np.tril(P, -1), np.tril(ref, -1))])
+    u, p = np.mean(ours, 0), np.mean(plain, 0)
+    assert u[0] < 0.75 * p[0] and u[1] < p[1], (u, p)
