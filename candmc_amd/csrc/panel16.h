@@ -643,27 +643,32 @@ struct Panel16 {
 
 // Products with a published panel: Vk holds its vectors as 16×16 tiles in
 // LDS (row-major, tile row i, pitch P16_LD), a[0..N) the caller's strip.
-// acc (16×16) += Σ_t V_tᵀ·a_t over tiles t < nact (tiles past nact are zero).
+// acc (16×16) + Σ_t V_tᵀ·a_t over tiles t < nact (tiles past nact are zero).
+// Four tiles at a time are summed from zero and then added: one chain over all
+// rows would round 4·N times at the size of its sum.
 template <int N>
 __device__ __forceinline__ dbl4 p16_vta(const double* __restrict__ Vk, const dbl4 (&a)[N], int nact, dbl4 acc, int lane) {
   const double* vp = Vk + (lane >> 4) * P16_LD + (lane & 15);
-  dbl4 acc2 = {0.0, 0.0, 0.0, 0.0};
+  dbl4 s0 = {0.0, 0.0, 0.0, 0.0}, s1 = s0;
 #pragma unroll
   for (int q = 0; q < (N + 3) / 4; ++q)
     if (q == 0 || 4 * q < nact) {
+      const dbl4 r0 = s0, r1 = s1;
+      s0 = s1 = dbl4{0.0, 0.0, 0.0, 0.0};
 #pragma unroll
       for (int t = 4 * q; t < 4 * q + 4; ++t)
         if (t < N) {
 #pragma unroll
           for (int v = 0; v < 4; ++v) {
             const double x = vp[t * P16_TILE + 4 * v * P16_LD];
-            if (v & 1) acc2 = __builtin_amdgcn_mfma_f64_16x16x4f64(x, a[t][v], acc2, 0, 0, 0);
-            else acc = __builtin_amdgcn_mfma_f64_16x16x4f64(x, a[t][v], acc, 0, 0, 0);
+            if (v & 1) s1 = __builtin_amdgcn_mfma_f64_16x16x4f64(x, a[t][v], s1, 0, 0, 0);
+            else s0 = __builtin_amdgcn_mfma_f64_16x16x4f64(x, a[t][v], s0, 0, 0, 0);
           }
         }
+      if (q > 0) acc += r0 + r1;
       __builtin_amdgcn_sched_barrier(0);   // sixteen operand loads ahead, no more registers than that
     }
-  return acc + acc2;
+  return acc + (s0 + s1);
 }
 
 // a_t += V_t·u over tiles t < nact (u: 16×16, tile layout).
