@@ -394,7 +394,7 @@ __global__ void __launch_bounds__(64) small_gemm_kernel(SmallArgs g) {
   const int i0 = blockIdx.x * 16, j0 = blockIdx.y * 16;
   // the operands of 128 values of k are in flight before the first is used
   const int c = lane & 15, q = lane >> 4, ia = i0 + c, jb = j0 + c;
-  dbl4 acc0 = {0.0, 0.0, 0.0, 0.0}, acc1 = acc0;
+  dbl4 acc = {0.0, 0.0, 0.0, 0.0};
   for (int k0 = 0; k0 < g.k; k0 += 128) {
     double x[32], y[32];
 #pragma unroll
@@ -403,17 +403,23 @@ __global__ void __launch_bounds__(64) small_gemm_kernel(SmallArgs g) {
       x[s] = g.A[ia < g.m && kk < g.k ? (g.ta ? kk + ia * g.lda : ia + kk * g.lda) : 0];
       y[s] = g.B[jb < g.n && kk < g.k ? (g.tb ? jb + kk * g.ldb : kk + jb * g.ldb) : 0];
     }
+    // 64 values at a time, two chains of 32 from zero
+    dbl4 s0 = {0.0, 0.0, 0.0, 0.0}, s1 = s0;
 #pragma unroll
     for (int s = 0; s < 32; ++s) {
+      if (s == 16) {
+        acc += s0 + s1;
+        s0 = s1 = dbl4{0.0, 0.0, 0.0, 0.0};
+      }
       if (k0 + 4 * s >= g.k) continue;
       const int kk = k0 + 4 * s + q;
       const double a = ia < g.m && kk < g.k ? gmask(x[s], g.ta ? kk : ia, g.ta ? ia : kk, g.smA) : 0.0;
       const double b = jb < g.n && kk < g.k ? gmask(y[s], g.tb ? jb : kk, g.tb ? kk : jb, g.smB) : 0.0;
-      if (s & 1) acc1 = __builtin_amdgcn_mfma_f64_16x16x4f64(b, a, acc1, 0, 0, 0);
-      else acc0 = __builtin_amdgcn_mfma_f64_16x16x4f64(b, a, acc0, 0, 0, 0);
+      if (s & 1) s1 = __builtin_amdgcn_mfma_f64_16x16x4f64(b, a, s1, 0, 0, 0);
+      else s0 = __builtin_amdgcn_mfma_f64_16x16x4f64(b, a, s0, 0, 0, 0);
     }
+    acc += s0 + s1;
   }
-  const dbl4 acc = acc0 + acc1;
   const int i = i0 + (lane & 15);
 #pragma unroll
   for (int v = 0; v < 4; ++v) {

@@ -137,3 +137,23 @@ def test_leaf_r(Q, m, b):
         ours.append(err(np.triu(Q.from_gpu(dA, m, b)[:b]), ref))
         plain.append(err(r_of(A), ref))
     assert np.mean(ours) < 0.88 * np.mean(plain), (np.mean(ours), np.mean(plain))
+
+
+@pytest.mark.parametrize("k", [128, 256])
+def test_small_product(Q, k):
+    """Y1ᵀ·Y2 of positive entries (sums that only grow): at most 1.35 times the
+    error of four running FP64 sums added up at the end."""
+    ours, plain = [], []
+    for seed in SEEDS:
+        print("small product", k, seed, flush=True)
+        A, B = np.abs(rnd(k, 32, seed)), np.abs(rnd(k, 32, seed + 9))
+        ref = A.T.astype(X) @ B.astype(X)
+        sums = [np.zeros((32, 32)) for _ in range(4)]
+        for i in range(k):
+            j = i // 4 % 4
+            sums[j] = (sums[j].astype(X) + np.outer(A[i].astype(X), B[i].astype(X))).astype(np.float64)
+        plain.append(err((sums[0] + sums[1]) + (sums[2] + sums[3]), ref))
+        dT = zeros(32 * 32)
+        Q.compute_invT_from_Y2(Q.to_gpu(np.asfortranarray(A)), k, Q.to_gpu(np.asfortranarray(B)), k, dT, 32, k, 32, 32)
+        ours.append(err(Q.from_gpu(dT, 32, 32), ref))
+    assert np.mean(ours) < 1.35 * np.mean(plain), (np.mean(ours), np.mean(plain))
