@@ -569,27 +569,9 @@ int run_chunks(cqr_ctx* c, LsqBatchPlan& P, int64_t np, const cqr_request* rq, c
   return CQR_OK;
 }
 
-}  // namespace
-
-size_t cqr_lstsq_batched_workspace_bytes(int64_t nprob, const cqr_request* reqs) {
-  if (nprob < 1 || !reqs) return 0;
-  for (int64_t p = 0; p < nprob; ++p) {
-    const cqr_request& r = reqs[p];
-    if (r.n < 1 || r.n > CQR_MAX_B || r.m < r.n || r.nrhs < 1 || r.nrhs > 16) return 0;
-  }
-  cqr_ctx dummy;   // planning only: set_err needs somewhere to write
-  LsqBatchPlan P;
-  if (plan_lsq_batch(&dummy, nprob, reqs, P) != CQR_OK) return 0;
-  return P.bytes;
-}
-
-int cqr_lstsq_batched(cqr_ctx* c, int64_t nprob, const cqr_request* reqs, int max_iter, double tol, int* status,
-                      int* iters, double* last_update) {
-  CQR_CHECK_CTX(c);
-  if (nprob < 1 || !reqs || !status || max_iter < 0 || !(tol >= 0.0))
-    return set_err(c, CQR_ERR_INVALID, "lstsq_batched: bad arguments");
-  LsqBatchPlan P;
-  CQR_TRY(plan_lsq_batch(c, nprob, reqs, P));
+// The whole call on planned requests; status[p] of the settled ones.
+int run_lsq_batch(cqr_ctx* c, LsqBatchPlan& P, int64_t nprob, const cqr_request* reqs, int max_iter, double tol,
+                  int* status, int* iters, double* last_update) {
   CQR_TRY(ensure_ws(c, P.bytes));
   char* base = static_cast<char*>(c->ws);
   cqr_batch& bt = P.bt;
@@ -613,9 +595,7 @@ int cqr_lstsq_batched(cqr_ctx* c, int64_t nprob, const cqr_request* reqs, int ma
     for (int64_t p = 0; p < nprob; ++p)
       CQR_TRY(launch_copy2d(c, reqs[p].A, reqs[p].lda, Ap + bt.aoff[p], bt.m[p], bt.m[p], bt.n[p]));
   }
-  int rc = CQR_OK;
-  for (Group& g : bt.groups)
-    if ((rc = run_group(c, &bt, g, Ap, Tp)) != CQR_OK) break;
+  for (Group& g : bt.groups) CQR_TRY(run_group(c, &bt, g, Ap, Tp));
   auto alone = [&](int64_t p) {
     const cqr_request& r = reqs[p];
     LsqRun run;
@@ -626,46 +606,74 @@ int cqr_lstsq_batched(cqr_ctx* c, int64_t nprob, const cqr_request* reqs, int ma
     if (iters) iters[p] = run.iters;
     if (last_update) last_update[p] = run.rel;
   };
-  if (rc != CQR_OK) {
-    for (int64_t p = 0; p < nprob; ++p) {
-      status[p] = rc;
-      if (iters) iters[p] = 0;
-      if (last_update) last_update[p] = 0.0;
-    }
-  } else if (apart) {
-    std::vector<LsqState> st;
-    CQR_TRY(run_chunks(c, P, nprob, reqs, base, true, [&](const LsqChunk& k) {
-      const int np = (int)(k.p1 - k.p0);
-      st.resize(np);
-      CQR_TRY(launch_lsq_solve(c, k.probs, k.states, np, k.nslab, k.nmax, 0, tol));
-      // two steps between looks at the states: most requests need no third
-      for (int it = 1;; it += 2) {
-        for (int i = it; i < it + 2 && i <= max_iter; ++i)
-          CQR_TRY(launch_lsq_solve(c, k.probs, k.states, np, k.nslab, k.nmax, i, tol));
-        CQR_HIP(c, hipMemcpyAsync(st.data(), k.states, sizeof(LsqState) * np, hipMemcpyDeviceToHost, c->stream));
-        CQR_HIP(c, hipStreamSynchronize(c->stream));
-        bool active = false;
-        for (const LsqState& x : st) active |= x.state == LSQ_ACTIVE;
-        if (!active || it + 2 > max_iter) break;
-      }
-      for (int64_t p = k.p0; p < k.p1; ++p) {
-        const LsqState& x = st[p - k.p0];
-        if (x.state == LSQ_DONE || (max_iter == 0 && x.state == LSQ_ACTIVE)) {
-          status[p] = CQR_OK;
-          if (iters) iters[p] = x.iters;
-          if (last_update) last_update[p] = x.rel;
-        } else {
-          alone(p);
-        }
-      }
-      return (int)CQR_OK;
-    }));
-  } else {
+  if (!apart) {
     for (int64_t p = 0; p < nprob; ++p) alone(p);
+    return CQR_OK;
   }
-  for (Group& g : bt.groups) g.d_bp = nullptr;   // arena memory, not owned
-  bt.ws = nullptr;
-  CQR_HIP(c, hipStreamSynchronize(c->stream));
+  std::vector<LsqState> st;
+  return run_chunks(c, P, nprob, reqs, base, true, [&](const LsqChunk& k) {
+    const int np = (int)(k.p1 - k.p0);
+    st.resize(np);
+    CQR_TRY(launch_lsq_solve(c, k.probs, k.states, np, k.nslab, k.nmax, 0, tol));
+    // two steps between looks at the states: most requests need no third
+    for (int it = 1;; it += 2) {
+      for (int i = it; i < it + 2 && i <= max_iter; ++i)
+        CQR_TRY(launch_lsq_solve(c, k.probs, k.states, np, k.nslab, k.nmax, i, tol));
+      CQR_HIP(c, hipMemcpyAsync(st.data(), k.states, sizeof(LsqState) * np, hipMemcpyDeviceToHost, c->stream));
+      CQR_HIP(c, hipStreamSynchronize(c->stream));
+      bool active = false;
+      for (const LsqState& x : st) active |= x.state == LSQ_ACTIVE;
+      if (!active || it + 2 > max_iter) break;
+    }
+    for (int64_t p = k.p0; p < k.p1; ++p) {
+      const LsqState& x = st[p - k.p0];
+      if (x.state == LSQ_DONE || (max_iter == 0 && x.state == LSQ_ACTIVE)) {
+        status[p] = CQR_OK;
+        if (iters) iters[p] = x.iters;
+        if (last_update) last_update[p] = x.rel;
+      } else {
+        alone(p);
+      }
+    }
+    return (int)CQR_OK;
+  });
+}
+
+}  // namespace
+
+size_t cqr_lstsq_batched_workspace_bytes(int64_t nprob, const cqr_request* reqs) {
+  if (nprob < 1 || !reqs) return 0;
+  for (int64_t p = 0; p < nprob; ++p) {
+    const cqr_request& r = reqs[p];
+    if (r.n < 1 || r.n > CQR_MAX_B || r.m < r.n || r.nrhs < 1 || r.nrhs > 16) return 0;
+  }
+  cqr_ctx dummy;   // planning only: set_err needs somewhere to write
+  LsqBatchPlan P;
+  if (plan_lsq_batch(&dummy, nprob, reqs, P) != CQR_OK) return 0;
+  return P.bytes;
+}
+
+int cqr_lstsq_batched(cqr_ctx* c, int64_t nprob, const cqr_request* reqs, int max_iter, double tol, int* status,
+                      int* iters, double* last_update) {
+  CQR_CHECK_CTX(c);
+  if (nprob < 1 || !reqs || !status || max_iter < 0 || !(tol >= 0.0))
+    return set_err(c, CQR_ERR_INVALID, "lstsq_batched: bad arguments");
+  LsqBatchPlan P;
+  CQR_TRY(plan_lsq_batch(c, nprob, reqs, P));
+  for (int64_t p = 0; p < nprob; ++p) {
+    status[p] = -1;   // not settled yet
+    if (iters) iters[p] = 0;
+    if (last_update) last_update[p] = 0.0;
+  }
+  int rc = run_lsq_batch(c, P, nprob, reqs, max_iter, tol, status, iters, last_update);
+  // an error ends the whole call: every request it left open gets it
+  for (int64_t p = 0; p < nprob; ++p)
+    if (status[p] < 0) status[p] = rc;
+  for (Group& g : P.bt.groups) g.d_bp = nullptr;   // arena memory, not owned
+  P.bt.ws = nullptr;
+  // (the tables stay until nothing can be on its way to the device)
+  if (hipStreamSynchronize(c->stream) != hipSuccess && rc == CQR_OK)
+    rc = set_err(c, CQR_ERR_DEVICE, "lstsq_batched: %s", hipGetErrorString(hipGetLastError()));
   return rc;
 }
 
