@@ -161,11 +161,12 @@ __device__ __forceinline__ void p16_fma_bc(double& acc, double z, double t) {
   asm("v_fmac_f64_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf" : "+&v"(acc) : "v"(z), "v"(t), "n"(C));
 }
 
-// sqrt and the two reciprocals of dlarfg for ss = ‖x‖² in (2^-960, 2^960)
-// and |alpha| < 2^480: beta = −sign(alpha)·sqrt(alpha² + ss) by the
-// Goldschmidt iteration from the hardware's reciprocal square root with two
-// residual corrections; no operand scaling is needed in this range (the
-// residual g² − x is a multiple of 2^-1064, and 1/beta at most 2^480).
+// sqrt and the two reciprocals of dlarfg for ss = ‖x‖² above 2^-960 and
+// alpha² + ss below overflow (tau is NaN beyond it): beta =
+// −sign(alpha)·sqrt(alpha² + ss) by the Goldschmidt iteration from the
+// hardware's reciprocal square root with two residual corrections; no operand
+// scaling is needed in this range (the residual g² − x is a multiple of
+// 2^-1064, and 1/beta at most 2^480).
 __device__ __forceinline__ void p16_larfg(double alpha, double ss, double& beta, double& tau, double& scal, double& rb) {
   const double x = fma(alpha, alpha, ss);
   const double y = __builtin_amdgcn_rsq(x);
@@ -224,15 +225,8 @@ struct Panel16 {
   static constexpr int H = PARTS > 1 ? RT : RT > 8 ? 8 : RT > 4 ? 4 : RT;
   double pr[P16];          // pivot rows
   double tau, scale;
-  double ssv, alv;         // what decides the fast range: ‖x‖² and alpha per column
+  uint32_t ssmin;          // the smallest high word of a column's ‖x‖² (see factor()), less one
 
-  // The fast range: ‖x‖² in (2^-960, 2^960) or x = 0, |alpha| < 2^480; a NaN
-  // or infinity fails it.  Dots of two columns in range stay below 2^960 and
-  // lose nothing to underflow that counts (2^-1074 against 2^-960); one that
-  // overflows makes its column infinite, which that column's own step shows.
-  __device__ static __forceinline__ bool in_range(double ss, double alpha) {
-    return ((ss > 0x1p-960 && ss < 0x1p960) || ss == 0.0) && fabs(alpha) < 0x1p480;
-  }
   // part ≠ 0, opaque as nact in column()
   __device__ __forceinline__ bool low() const {
     int p = part;
@@ -298,7 +292,10 @@ struct Panel16 {
     const double ss = readlane_d(s, J), alpha = readlane_d(p, J);
     // a column without anything below its diagonal: H = I (by masks alone, as
     // the values of p16_larfg then need not be numbers)
-    const int cj = (__double2loint(ss) | __double2hiint(ss)) != 0 ? J : P16;
+    int sh = __double2hiint(ss);
+    asm("" : "+s"(sh));                         // (tested in scalar registers)
+    const int cj = sh != 0 ? J : P16;
+    ssmin = min(ssmin, (uint32_t)sh - 1u);
     double beta, tj, scal, rb;
     p16_larfg(alpha, ss, beta, tj, scal, rb);
     const double wv = fma(scal, s, p);          // v_Jᵀ·(column c), v_J = [1; scal·x]
@@ -318,8 +315,6 @@ struct Panel16 {
       pr[J] = c > cj ? fma(-tj, wv, p) : (c == cj ? beta : p);
       Zc[J * P16_LD] = wv * scale * -tj;        // four lanes, one value
     }
-    ssv = c == J ? s : ssv;
-    alv = c == J ? p : alv;
     tau = c == cj ? tj : tau;
     scale = c == cj ? scal : scale;
   }
@@ -448,7 +443,7 @@ struct Panel16 {
       const double ss = readlane_d(s, j), alpha = readlane_d(p, j);
       m = readlane_d(m, j);
       double beta, tj, fs, sc, wv;                // sc: the vector's scale, fs: the update's factor
-      if (ss != 0.0 && in_range(ss, alpha)) {
+      if (ss > 0x1p-960 && ss < 0x1p960 && fabs(alpha) < 0x1p480) {
         p16_larfg(alpha, ss, beta, tj, sc, fs);
         wv = fma(sc, s, p);
       } else {
@@ -549,7 +544,7 @@ struct Panel16 {
     const int c = lane & 15;
     tau = 0.0;
     scale = 1.0;
-    ssv = alv = 1.0;
+    ssmin = ~0u;
     // the strip may come straight from MFMAs, whose results the inline VALU
     // code below must not read before they land
     __builtin_amdgcn_sched_barrier(0);
@@ -577,8 +572,13 @@ struct Panel16 {
     P16_STEP(8) P16_STEP(9) P16_STEP(10) P16_STEP(11) P16_STEP(12) P16_STEP(13) P16_STEP(14) P16_STEP(15)
 #undef P16_STEP
     int bar = 0;
-    bool redo = __builtin_amdgcn_ballot_w64(!in_range(ssv, alv)) != 0;
-    if (const uint64_t z = __builtin_amdgcn_ballot_w64(ssv == 0.0)) {
+    // Exact as they stand are columns with ‖x‖² above 2^-960 (dots of two of
+    // them lose nothing to underflow that counts, 2^-1074 against 2^-960) and
+    // no overflow, which makes its column infinite and that column's tau NaN,
+    // as a NaN or an infinity in the data does, and columns with x = 0.
+    bool redo = __builtin_amdgcn_ballot_w64(tau != tau) != 0 || ssmin < 0x03f00000u;
+    const uint64_t zero = __builtin_amdgcn_ballot_w64(tau == 0.0 && c < nb);
+    if (__builtin_expect(zero != 0, 0)) {
       // really nothing there, or entries too small to square?  (they are as
       // their column's own step found them)
       double nz = 0.0;
@@ -589,7 +589,7 @@ struct Panel16 {
       if (!NODE)
 #pragma unroll
         for (int q = 0; q < P16; ++q) nz = fmax(nz, (PARTS > 1 && part != 0 ? q < 4 : q > c) ? fabs(pr[q]) : 0.0);
-      bool some = __builtin_amdgcn_ballot_w64(ssv == 0.0 && nz > 0.0) != 0;
+      bool some = __builtin_amdgcn_ballot_w64(tau == 0.0 && nz > 0.0) != 0;
       if constexpr (PARTS > 1) {                  // one decision for all parts
         double* E = ex + 2 * P16 * (PARTS + 1);
         if (lane == 0) {
@@ -606,7 +606,7 @@ struct Panel16 {
       redo |= some;
       if (PARTS == 1 || part == 0)
         for (int q = 0; q < P16; ++q)
-          if (z >> q & 1) Zc[q * P16_LD] = 0.0;
+          if (zero >> q & 1) Zc[q * P16_LD] = 0.0;
     }
     if constexpr (GLOB)   // (without meaning if the panel is redone)
 #pragma unroll

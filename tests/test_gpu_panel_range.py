@@ -156,3 +156,31 @@ def test_general_route_is_not_much_slower(Q, m, b, kind):
 
     us(A)
     assert us(Z) < 4 * us(A)
+
+
+@pytest.mark.parametrize("e", [-474, 505])
+@pytest.mark.parametrize("m,b", LEAVES)
+def test_scaled_to_the_ends(Q, m, b, e):
+    """As far as a column's ‖x‖² neither falls below 2^-960 nor overflows."""
+    A = O.gaussian(m, b, m + b)
+    YR, T, tau = leaf(Q, A)
+    YS, TS, ts = leaf(Q, np.ldexp(A, e))
+    assert np.array_equal(T, TS) and np.array_equal(tau, ts)
+    assert np.array_equal(np.tril(YR, -1), np.tril(YS, -1))
+    assert np.array_equal(np.ldexp(np.triu(YR[:b]), e), np.triu(YS[:b]))
+
+
+@pytest.mark.parametrize("e", [-560, 509, 700])
+@pytest.mark.parametrize("m,b", [(256, 16), (256, 128), (512, 64), (1000, 16)])
+def test_one_column_past_the_ends(Q, m, b, e):
+    """A column whose ‖x‖² underflows or overflows sends its strip the general
+    way; the result is that of the unscaled matrix to rounding."""
+    A = O.gaussian(m, b, m + b)
+    d = np.zeros(b, int)
+    d[b - 3] = e
+    YR, T, tau = leaf(Q, A)
+    YS, TS, ts = leaf(Q, np.ldexp(A, d))
+    tol = 64 * m * EPS
+    assert np.abs(T - TS).max() < tol * b and np.abs(tau - ts).max() < tol
+    assert np.abs(np.tril(YR, -1) - np.tril(YS, -1)).max() < tol * b
+    assert np.abs(np.triu(YR[:b]) - np.ldexp(np.triu(YS[:b]), -d)).max() < tol * np.abs(YR[:b]).max()
