@@ -285,8 +285,9 @@ int bgemm(cqr_ctx* c, const BgemmArgs& g, int batch, int max_m);
 // Householder reconstruction of a panel's top block (hr_kernel.hip, b ≤ 128):
 // signed LU of Q1top − S; Atop := [L \\ S·R], W = U·S, U⁻¹ (ld b, zeros below
 // the diagonal), and whichever of the others are non-null: the signs, Tᵀ, T,
-// T⁻ᵀ (all ld b, zeros outside their triangle), M2 = U⁻¹·Tᵀ (needs Tt), and
-// the top b rows of the explicit Y and of Y·Tᵀ (ld ldy).
+// T⁻ᵀ (all ld b, zeros outside their triangle; T⁻ᵀ needs Uinv), M2 = U⁻¹·Tᵀ
+// (needs Tt and Uinv), and the top b rows of the explicit Y and of Y·Tᵀ (ld
+// ldy).
 struct HrCore {
   const double* Q1top;
   int64_t ldq;

@@ -351,7 +351,7 @@ struct HrArgs {
   int64_t* signs;
   double* Tt;          // Tᵀ = −L⁻¹·Wᵀ
   double* T;
-  double* invTT;       // T⁻ᵀ = −W⁻ᵀ·L
+  double* invTT;       // T⁻ᵀ = −W⁻ᵀ·L (needs Uinv)
   double* M2;          // U⁻¹·Tᵀ (needs Tt)
   double* Ye;          // top rows of the explicit Y and of Y·Tᵀ = −Wᵀ there
   double* YT;
@@ -361,7 +361,8 @@ struct HrArgs {
 
 }  // namespace
 
-// Everything but Q1top, Rroot, Atop and W may be null.
+// Everything but Q1top, Rroot, Atop and W may be null; M2 needs Tt and Uinv,
+// invTT needs Uinv (U⁻¹'s tiles are formed for it only).
 template <int W>
 __device__ __forceinline__ void hr16_body(const HrArgs& h, double* smem) {
   const int lane = threadIdx.x & 63, s = strip_of<W>(wave_id());
@@ -597,6 +598,7 @@ int hr_core(cqr_ctx* c, const HrCore& a) {
   const int b = a.b;
   if (b < 1 || b > 128) return set_err(c, CQR_ERR_UNSUPPORTED, "hr_core: b = %d", b);
   if (a.M2 && !(a.Tt && a.Uinv)) return set_err(c, CQR_ERR_INVALID, "hr_core: M2 needs Tt and Uinv");
+  if (a.invTT && !a.Uinv) return set_err(c, CQR_ERR_INVALID, "hr_core: invTT needs Uinv");
   HrArgs h{};
   h.Q1top = a.Q1top; h.ldq = a.ldq; h.Rroot = a.Rroot; h.Atop = a.Atop; h.lda = a.lda; h.W = a.W; h.Uinv = a.Uinv;
   h.signs = a.signs; h.Tt = a.Tt; h.T = a.T; h.invTT = a.invTT; h.M2 = a.M2; h.Ye = a.Ye; h.YT = a.YT; h.ldy = a.ldy;
