@@ -154,11 +154,10 @@ int make_plan(int64_t m, int64_t b, int64_t nleaves_hint, int64_t leaf_rows,
 // Batched small GEMM addressing: batch index z selects each operand as
 //   BM_STRIDED  p + z·zs          (per-leaf / per-node b×b arrays)
 //   BM_LEAFROWS p + rowoff(z)     (leaf z's rows inside a column-major panel)
-//   BM_SHIFTED  p + (z+zoff)·zs   (the sender of tree pair z)
 //   BM_LEAFROWS_SHIFTED p + rowoff(z+zoff)  (the sender's rows of tree pair z)
 // m < 0 or k < 0 stands for the rows of leaf z.
 // ---------------------------------------------------------------------------
-enum { BM_STRIDED = 0, BM_LEAFROWS = 1, BM_SHIFTED = 2, BM_LEAFROWS_SHIFTED = 3 };
+enum { BM_STRIDED = 0, BM_LEAFROWS = 1, BM_LEAFROWS_SHIFTED = 2 };
 struct BMat {
   const double* p;
   int64_t ld;
@@ -172,7 +171,7 @@ struct BgemmArgs {
   double alpha, beta;
   int64_t pm;             // panel rows for BM_LEAFROWS / m < 0
   int pL;                 // leaves
-  int zoff;               // for BM_SHIFTED
+  int zoff;               // for BM_LEAFROWS_SHIFTED
 };
 inline BMat bmat(const double* p, int64_t ld, int64_t zs = 0, int mode = BM_STRIDED) {
   BMat b; b.p = p; b.ld = ld; b.zs = zs; b.mode = mode; return b;
@@ -264,7 +263,8 @@ int update_y_batched(cqr_ctx* c, const BatchProb* bp, const BatchSeg* seg, int n
 // and U⁻¹ b×b per problem, Tᵀ at the problem's toff.
 int hr_core_batched(cqr_ctx* c, const BatchProb* bp, int nprob, const double* Y, const double* leafR,
                     const double* nodeR, double* Abase, double* W, double* Uinv, double* Tt, int b);
-// Leaves of 64 < b ≤ 128 columns and at most 256 rows (ptree_kernel.hip)
+// Leaf QR of every row block (ptree_kernel.hip): leaves of at most 1024 rows at
+// b ≤ 32, 512 at b ≤ 64, 256 at b ≤ 128 (rows: the largest leaf)
 int leaf16(cqr_ctx* c, double* A, int64_t lda, int64_t m, int L, int64_t rows, int b, double* R, double* T, double* tau,
            const BatchProb* bp, int nprob);
 

@@ -21,7 +21,7 @@
 //
 // Bound: the serial chain of b columns (one recip and one broadcast FMA per
 // tile row each), then MFMA issue on one CU.  At b = 128 with Tᵀ and U⁻¹·Tᵀ
-// 88–100 µs, b = 64 40 µs, b = 32 15 µs; the form before (8-column steps
+// 88–100 µs, b = 64 37 µs, b = 32 15 µs; the form before (8-column steps
 // through LDS, in-place inverses one after the other) took 160–210, 75 and
 // 47 µs and left T, T⁻ᵀ, and below b = 128 Tᵀ, U⁻¹·Tᵀ and the top rows of
 // Y and Y·Tᵀ, to small products of 6–20 µs each.

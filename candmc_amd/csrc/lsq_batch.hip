@@ -18,8 +18,8 @@
 // Bound: the chains inside a workgroup (a slab's rows one after another, the
 // solve's sixteen tile steps), then HBM.  32 requests of 64 columns, rows
 // around 4096 and 1 to 16 right-hand sides: 7.3 ms with a chain of a hundred
-// small launches and a synchronisation per step and request, 0.98 ms so, of
-// it the factorization 0.6 ms, a slab launch 55 (Yᵀb) or 83 µs (Aᵀ(b − A·x)),
+// small launches and a synchronisation per step and request, 0.92 ms so, of
+// it the factorization 0.57 ms, a slab launch 55 (Yᵀb) or 83 µs (Aᵀ(b − A·x)),
 // a solve 30 µs.
 #include "cqr_device.h"
 #include "cqr_internal.h"

@@ -328,10 +328,9 @@ struct Panel16 {
   // left (entries too far apart, NaN, infinities) takes up to three more passes
   // and dlarfg_scalar.  Two passes a column, two or four tiles in flight; keeping
   // the strip in the registers that are free here spilled in the straight-line
-  // steps.  hh_recon_qr with every entry around 1e-200: 256×16 130 µs (78 in
-  // range), 32768×128 1220 (498), 65536×16 480 (187); with one value in
-  // flight, a division an element and one wave for a whole tall leaf 372, 3600 and
-  // 4470.
+  // steps.  hh_recon_qr with every entry around 1e-200: 256×16 100 µs (49 in
+  // range), 32768×128 1030 (460), 65536×16 420 (147); with one value in flight,
+  // a division an element and one wave for a whole tall leaf 347, 3540 and 4400.
   __device__ __forceinline__ double slow(double* Vs, double* Ds, double* Zs, int nt, int nb, int& bar) const {
     const int lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
     const bool first = PARTS == 1 || part == 0;   // holds the pivot tile

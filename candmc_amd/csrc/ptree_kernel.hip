@@ -28,9 +28,10 @@
 // the next strip's products); a tree level adds about 13 µs.  Before, with
 // one reflector at a time broadcast through LDS (leaf) and 8-column blocks
 // with four products and six barriers each (node), a leaf took 0.25–0.30 ms
-// and a level 21 µs: hh_recon_qr of 32768×128 0.88 → 0.67 ms, of 4099×100
-// (a width that took a column-at-a-time node) 0.94 → 0.44 ms, 512 batched
-// problems of up to 16384×128 17.5 → 13.8 ms, QR 32768×4096 43.9 → 38.2 ms.
+// and a level 21 µs: with this and the other kernels' gains hh_recon_qr of
+// 32768×128 went 0.88 → 0.49 ms, of 4099×100 (a width that took a
+// column-at-a-time node) 0.95 → 0.34 ms, 512 batched problems of up to
+// 16384×128 17.4 → 10.4 ms, QR 32768×4096 43.9 → 33.0 ms.
 #include "cqr_device.h"
 #include "cqr_internal.h"
 #include "panel16.h"
@@ -252,10 +253,10 @@ __device__ __forceinline__ void leaf16_body(double* __restrict__ A, int64_t lda,
 // one panel of V in LDS.  Three loops rather than one with roles: the factor()
 // of the strip's own panel then stands in no loop, where its registers
 // spilled.  512×64 leaves take 0.11 ms (0.125 with a reflector at a time over
-// 64-row lanes); hh_recon_qr of 65536×16 234 → 153 µs, ×32 328 → 245,
-// 16384×64 458 → 321 (with the other kernels' gains).  A single strip (b ≤ 16)
+// 64-row lanes); hh_recon_qr of 65536×16 225 → 147 µs, ×32 321 → 234,
+// 8192×64 416 → 275 (with the other kernels' gains).  A single strip (b ≤ 16)
 // keeps its vectors in registers, so that two or four leaves share a CU: 4500
-// leaves of 1024×16 take 0.46 ms, 0.70 with V in 143 KB of LDS, a leaf a CU.
+// leaves of 1024×16 take 0.43 ms, 0.70 with V in 143 KB of LDS, a leaf a CU.
 // ---------------------------------------------------------------------------
 template <int S, int P>
 constexpr int tall_smem_doubles() {

@@ -208,10 +208,9 @@ tree_node_kernel(double* __restrict__ Rleaf, int n, int node0, int b, double* __
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ const double* bmat_ptr(const BMat& M, int z, const BgemmArgs& g) {
   switch (M.mode) {
-    case BM_STRIDED: return M.p + (int64_t)z * M.zs;
     case BM_LEAFROWS: return M.p + leaf_off(z, g.pm, g.pL);
     case BM_LEAFROWS_SHIFTED: return M.p + leaf_off(z + g.zoff, g.pm, g.pL);
-    default: return M.p + (int64_t)(z + g.zoff) * M.zs;
+    default: return M.p + (int64_t)z * M.zs;   // BM_STRIDED
   }
 }
 
